@@ -313,6 +313,41 @@ def test_fast_prefill_climbing_scores(torch_cuda):
     assert np.array_equal(one[-1].view(np.uint32), three[-1].view(np.uint32))
 
 
+@pytest.mark.parametrize("group", [1, 2, 3, 4])
+def test_fast_prefill_rows_same_in_small_and_large_launches(torch_cuda, group):
+    """The prefill attention computes a KV head's query heads in separate
+    work-groups up to 512 (16-row block, KV head) items and together beyond:
+    a chunk of 41 rows (a ragged last block) at position 500 (36 pages for
+    eight page streams) alone (9 items) and beside nine sequences of 304
+    rows (522 items) gives bit-identical logits, within 1e-3 relative of the
+    oracle, for 1 to 4 query heads per KV head."""
+    h = 192 * group
+    cfg = dict(layers=1, hidden=h, intermediate=64, heads=3 * group, kv_heads=3, vocabulary=256, context=640, eos=0,
+               rms_epsilon=1e-5, rope_theta=100000.0, tied=0)
+    model = OracleModel(cfg, seed=71, stddev=0.05)
+    o = Oracle()
+    prompt = [int(t) for t in o.fill_tokens(541, 71, 9700, 256)]
+    others = [int(t) for t in o.fill_tokens(9 * 304, 71, 9701, 256)]
+    outs = []
+    for beside in (0, 9):
+        backend = HipBackend(cfg, block_tokens=16, max_blocks=400, max_sequences=10, arithmetic=ARITHMETIC_FAST)
+        upload_model(backend, model)
+        for i in range(10):
+            backend.table_write(i, 0, np.arange(40 * i, 40 * i + 40, dtype=np.int32)[::-1].copy())
+        backend.forward([(0, 0, 500)], prompt[:500])
+        _, got = backend.forward([(0, 500, 41)] + [(i, 0, 304) for i in range(1, 1 + beside)],
+                                 prompt[500:] + others[:304 * beside])
+        outs.append(got[0].copy())
+        backend.close()
+    n = pool_elements(cfg, 16, 40)
+    keys, values = np.zeros(n, np.float32), np.zeros(n, np.float32)
+    table = np.arange(40, dtype=np.int32)
+    model.append(keys, values, 16, table, 0, prompt[:500])
+    want = model.append(keys, values, 16, table, 500, prompt[500:])
+    assert rel_inf(outs[0], want) <= 1e-3
+    assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+
+
 def test_fast_small_batch_decode_gemv(torch_cuda):
     """Decode steps of up to four sequences take the GEMV projections
     (row-major weights, RMSNorm computed inside the projections): 90
