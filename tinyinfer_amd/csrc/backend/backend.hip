@@ -72,7 +72,7 @@ struct mp_hip {
     // the decode attention's split partials (grow-only).
     bool fast = false;
     float* ssq = nullptr;
-    int32_t* row_block = nullptr;  // [workspace rows]: page of each row's position (decode)
+    int32_t* row_block = nullptr;  // [workspace rows]: page of each row's position
     float* row_rope = nullptr;     // [workspace rows][head dim]: cos | sin at each row's position
     float* fast_partials = nullptr;
     size_t fast_partial_floats = 0;
@@ -803,7 +803,7 @@ int mp_hip_forward(mp_hip* h, const mp_seq_step* steps, int32_t nseq, const int3
     // splits (fast_attention_split); rows of up to 256 tokens as (row, KV
     // head, tokens) items of the one-work-group kernel; the rows the merge
     // kernel combines. The split depends on nothing but the row.
-    const bool fast_decode = fast_rows && decode;  // q|k|v with the RoPE epilogue
+    const bool fast_decode = fast_rows && decode;
     size_t fast_items = 0, fast_short = 0, fast_merge = 0, fast_pre = 0;
     int max_splits = 0;
     if (fast_rows)
@@ -1052,13 +1052,13 @@ int mp_hip_forward(mp_hip* h, const mp_seq_step* steps, int32_t nseq, const int3
         if (r == hipSuccess) r = gemm(epi, h->xn, rows, inner, w, w2, columns, out);
         return r;
     };
-    // The fast decode's q|k|v projection takes each row's page and rotation
-    // from per-row arrays that the embedding kernel fills.
+    // The fast q|k|v projection takes each row's page and rotation from
+    // per-row arrays that the embedding kernel fills.
     mphip::RowRope row_rope{meta, h->tables, h->kv.max_sequence_blocks, h->kv.block_tokens, dim / 2,
                             h->cos_table, h->sin_table, h->row_block, h->row_rope};
     auto launch_embedding = [&]() {
         return mphip::launch_embed(s, h->embedding, meta.tokens, h->x, R, hd, device_error,
-                                   fast_decode ? &row_rope : nullptr, h->fast);
+                                   fast_rows ? &row_rope : nullptr, h->fast);
     };
     // The fast arithmetic's launches from the embedding to the argmax; with
     // graph_grids the attention grids are sized by the lists' capacities, for
@@ -1152,8 +1152,11 @@ int mp_hip_forward(mp_hip* h, const mp_seq_step* steps, int32_t nseq, const int3
             layer_now = l;
             if (gemv_rows) {
                 e = timed(P, [&] { return gemv(mphip::kRope, h->x, hd, h->qkv_rows[l], nullptr, qw, h->qkv_out, h->input_norm[l], l); });
-            } else if (fast_decode) {
-                // q|k|v with RoPE and the KV append in the epilogue.
+            } else if (fast_rows) {
+                // q|k|v with RoPE and the KV append in the epilogue, in steps
+                // that prefill as well: a rope_append launch after a plain
+                // projection took 20.6 against 11.4 us at 256 rows and 105.6
+                // against 80.2 us at 4,096 (with the q|k|v projection).
                 e = timed(P, [&] {
                     mphip::FastGemmArgs a{};
                     a.x = h->x;
@@ -1189,13 +1192,9 @@ int mp_hip_forward(mp_hip* h, const mp_seq_step* steps, int32_t nseq, const int3
                                                             h->ctx, hd, fw);
                     });
                 } else if (fast_rows) {
-                    // RoPE and the K/V append of every row, then the prefill
-                    // rows; the one-token rows after them.
-                    e = mphip::launch_rope_append(s, h->qkv_out, qw, R, c.heads, c.kv_heads, dim, h->cos_table,
-                                                  h->sin_table, meta, kv, l);
-                    if (e == hipSuccess)
-                        e = mphip::launch_fast_prefill(s, h->qkv_out, qw, c.heads, c.kv_heads, kv, l,
-                                                       h->meta + pre_at, (int)fast_pre, h->ctx, hd);
+                    // The prefill rows; the one-token rows after them.
+                    e = mphip::launch_fast_prefill(s, h->qkv_out, qw, c.heads, c.kv_heads, kv, l, h->meta + pre_at,
+                                                   (int)fast_pre, h->ctx, hd);
                     if (e == hipSuccess && fast_items + fast_short > 0)
                         e = mphip::launch_fast_attention(s, h->qkv_out, qw, R, c.heads, c.kv_heads, meta, kv, l,
                                                          h->ctx, hd, fw);

@@ -40,7 +40,7 @@
 // the sum of squares of the updated x over each 16-column block; SwiGLU
 // (gate and up accumulated side by side); LM head (per row and column group
 // of 16*CB columns, the first maximum and a non-finite flag, logits
-// row-major on request); RoPE (the q|k|v projection of a decode step, over
+// row-major on request); RoPE (the q|k|v projection, over
 // q and k columns stored pair-permuted so that each 16-column block holds
 // whole split-half pairs (d, d+32) in lanes c and c+8; q is rotated in
 // place, the rotated k and the v go to the paged pools at the row's
@@ -103,7 +103,6 @@ __device__ __forceinline__ int rope_pair(int cb, int lane) { return 8 * (cb & 3)
 
 template <int EPI, bool NORM, bool GATHER, int RB, int CB, int CH>
 __global__ __launch_bounds__(kWaves * 64, CH == 1 ? 4 : 1) void fast_gemm_kernel(FastGemmArgs a) {
-    static_assert(EPI != kRope || CB == 1, "the RoPE epilogue takes one column block");
     constexpr int M = EPI == kSwiglu ? 2 : 1;
     constexpr int NB = CB * M;  // B operands per step
     constexpr int T = RB * NB;  // accumulator tiles
@@ -182,19 +181,27 @@ __global__ __launch_bounds__(kWaves * 64, CH == 1 ? 4 : 1) void fast_gemm_kernel
         }
     }
     // RoPE rows of the owned row block: position, page and rotation (cos,
-    // sin of rotation index rope_pair() at the row's position; CB == 1).
+    // sin of rotation index rope_pair() at the row's position). A tile of
+    // several column blocks (many rows) reads the rotations in the epilogue.
     int rope_pos[4], rope_block[4];
     float rope_cs[4], rope_sn[4];
+    auto load_rotation = [&](int j) {
+        const int rd = rope_pair(cblock[j], lane);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int row = min(row0 + wave * 16 + 4 * (lane >> 4) + i, a.rows - 1);
+            rope_cs[i] = a.row_rope[(size_t)row * kRopeDim + rd];
+            rope_sn[i] = a.row_rope[(size_t)row * kRopeDim + kRopeDim / 2 + rd];
+        }
+    };
     if (EPI == kRope && wave < OW) {
-        const int rd = rope_pair(cblock[0], lane);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int row = min(row0 + wave * 16 + 4 * (lane >> 4) + i, a.rows - 1);
             rope_pos[i] = a.meta.row_pos[row];
             rope_block[i] = a.row_block[row];
-            rope_cs[i] = a.row_rope[(size_t)row * kRopeDim + rd];
-            rope_sn[i] = a.row_rope[(size_t)row * kRopeDim + kRopeDim / 2 + rd];
         }
+        if (CB == 1) load_rotation(0);
     }
 
     f4 acc[T];
@@ -334,43 +341,47 @@ __global__ __launch_bounds__(kWaves * 64, CH == 1 ? 4 : 1) void fast_gemm_kernel
 
     const int N = a.columns;
     if (EPI == kRope) {
-        // One column block (CB == 1) of the pair-permuted q|k|v columns:
-        // lanes c and c + 8 of a q or k block hold the split-half pair
-        // (d, d + 32) of one head (rope_dim), exchanged by a DPP rotation of
-        // the 16-lane row by 8; v blocks are in natural order. RB <= 4, so
-        // wavefront w owns row block w.
+        // Column blocks of the pair-permuted q|k|v columns: lanes c and c + 8
+        // of a q or k block hold the split-half pair (d, d + 32) of one head
+        // (rope_dim), exchanged by a DPP rotation of the 16-lane row by 8; v
+        // blocks are in natural order. RB <= 4, so wavefront w owns row
+        // block w.
         const int rb = wave;
-        const int cb = cblock[0];
-        const int hcol = cb * 16 / kRopeDim * kRopeDim;  // the head's first column
         const int hidden = a.heads * kRopeDim, kvw = a.kv.kv_width;
         const int bt = a.kv.block_tokens;
-        const bool rotate = hcol < hidden + kvw;
-        const int d = rotate ? rope_dim(cb, lane) : (cb * 16) % kRopeDim + (lane & 15);
         const bool low = (lane & 8) == 0;  // the d < 32 half of a pair
-        float x[4], xp[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float v = 0.0f;
+        for (int j = 0; j < CB; ++j) {
+            const int cb = cblock[j];
+            const int hcol = cb * 16 / kRopeDim * kRopeDim;  // the head's first column
+            const bool rotate = hcol < hidden + kvw;
+            const int d = rotate ? rope_dim(cb, lane) : (cb * 16) % kRopeDim + (lane & 15);
+            if (CB > 1 && rotate) load_rotation(j);
+            float x[4], xp[4];
 #pragma unroll
-            for (int r2 = 0; r2 < RB; ++r2)
-                if (r2 == rb) v = acc[r2][i];
-            x[i] = v * inv_s[rb * 16 + 4 * (lane >> 4) + i];
-            xp[i] = dpp<kDppRowRor8>(x[i]);
-        }
+            for (int i = 0; i < 4; ++i) {
+                float v = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = row0 + rb * 16 + 4 * (lane >> 4) + i;
-            if (row >= a.rows) continue;
-            const float cs = rope_cs[i], sn = rope_sn[i];
-            const float y = !rotate ? x[i] : low ? x[i] * cs - xp[i] * sn : x[i] * cs + xp[i] * sn;
-            if (hcol < hidden) {
-                a.out[quad_index(row, hcol + d, N)] = y;
-                continue;
+                for (int r2 = 0; r2 < RB; ++r2)
+                    if (r2 == rb) v = acc[r2 * NB + j][i];
+                x[i] = v * inv_s[rb * 16 + 4 * (lane >> 4) + i];
+                xp[i] = dpp<kDppRowRor8>(x[i]);
             }
-            const size_t base = kv_page_base(rope_block[i], a.layer, a.kv.layers, bt, kvw);
-            const int slot = rope_pos[i] % bt;
-            if (rotate) a.kv.keys[base + key_offset(slot, (hcol - hidden) / kRopeDim, d, bt, kRopeDim)] = y;
-            else a.kv.values[base + value_offset(slot, (hcol - hidden - kvw) / kRopeDim, d, bt, kRopeDim)] = y;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int row = row0 + rb * 16 + 4 * (lane >> 4) + i;
+                if (row >= a.rows) continue;
+                const float cs = rope_cs[i], sn = rope_sn[i];
+                const float y = !rotate ? x[i] : low ? x[i] * cs - xp[i] * sn : x[i] * cs + xp[i] * sn;
+                if (hcol < hidden) {
+                    a.out[quad_index(row, hcol + d, N)] = y;
+                    continue;
+                }
+                const size_t base = kv_page_base(rope_block[i], a.layer, a.kv.layers, bt, kvw);
+                const int slot = rope_pos[i] % bt;
+                if (rotate) a.kv.keys[base + key_offset(slot, (hcol - hidden) / kRopeDim, d, bt, kRopeDim)] = y;
+                else a.kv.values[base + value_offset(slot, (hcol - hidden - kvw) / kRopeDim, d, bt, kRopeDim)] = y;
+            }
         }
         return;
     }
@@ -675,7 +686,8 @@ hipError_t launch_fast(hipStream_t s, const FastGemmArgs& a) {
 // give every CU a work-group: they read each weight and each activation a
 // quarter as often. Otherwise the largest of 64 x 16, 32 x 16 and 16 x 16
 // that gives every CU a work-group. (The q|k|v+RoPE projection keeps
-// 64 x 16 or 32 x 16 tiles above 64 rows: 11.2 vs 16.0 us at 256 rows.)
+// 64 x 16 or 32 x 16 tiles above 64 rows, 11.2 vs 16.0 us at 256 rows, up to
+// where 64 x 64 tiles give every CU a work-group.)
 constexpr int kCus = 256;
 bool head_wide(int columns) { return columns % 64 == 0; }
 int tiles(const FastGemmArgs& a, int rb, int cb) { return ((a.rows + 15) / 16 + rb - 1) / rb * (a.columns / 16 / cb); }
@@ -736,6 +748,7 @@ hipError_t launch_fast_gemm(hipStream_t s, Epilogue epilogue, const FastGemmArgs
         if (a.columns % kRopeDim || a.heads * kRopeDim + 2 * a.kv.kv_width != a.columns || !norm ||
             a.kv.block_tokens <= 0 || !a.row_block || !a.row_rope)
             return hipErrorInvalidValue;
+        if (a.rows > 256 && tiles(a, 4, 4) >= kCus) return launch_fast<kRope, true, false, 4, 4, 2>(s, a);
         if (a.rows > 64 && tiles(a, 4, 1) >= kCus) return launch_fast<kRope, true, false, 4, 1, 2>(s, a);
         if (a.rows > 64 && tiles(a, 2, 1) >= kCus) return launch_fast<kRope, true, false, 2, 1, 6>(s, a);
         return launch_fast<kRope, true, false, 1, 1, 12>(s, a);
