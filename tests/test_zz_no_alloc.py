@@ -63,3 +63,52 @@ def test_noalloc_matches_allocating_entry_point(torch_cuda):
     with pytest.raises(BackendError) as error:
         paged_attention_decode_noalloc(*long_args, out.data_ptr(), None)
     assert "exceeds" in str(error.value)
+
+
+def _check(torch, o, seed, length, heads, kv_heads, scale=1.0, equal_keys=False):
+    layers, layer = 2, 1
+    pages = math.ceil(length / BT) + 3
+    kvw = kv_heads * DIM
+    keys = o.fill_normal(pages * layers * BT * kvw, seed, 1)
+    if equal_keys:
+        keys[:] = 0.25
+    values = o.fill_normal(pages * layers * BT * kvw, seed, 2)
+    q = o.fill_normal(heads * DIM, seed, 3, scale)
+    table = o.permutation(pages, seed, 4)[: math.ceil(length / BT)].copy()
+    want = o.attention(q, keys, values, table, length - 1, 1, layer, layers, BT, heads, kv_heads, DIM)[0]
+    dq, dk, dv, dt = (torch.from_numpy(a).cuda() for a in (q, keys, values, table))
+    for call in (paged_attention_decode, paged_attention_decode_noalloc):
+        got = torch.full((heads * DIM,), float("nan"), dtype=torch.float32, device="cuda")
+        call(dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dt.data_ptr(), length, layer, layers, BT, heads, kv_heads, DIM,
+             got.data_ptr(), None)
+        torch.cuda.synchronize()
+        g = got.cpu().numpy()
+        assert np.array_equal(g.view(np.uint32), want.view(np.uint32)), (call.__name__, length, heads, kv_heads)
+
+
+@pytest.mark.parametrize("length", [1, 15, 17, 64, 224, 225, 256, 257, 511, 640, 641, 896, 897, 1025, 3413, 3414, 18431,
+                                    18432, 18433, 20000])
+def test_row_kernel_edges(torch_cuda, length):
+    """Bits of the oracle at the edges of the row kernel: partial pages,
+    phases of 14 pages and turns of four phases, the 256 denominator values
+    added one by one, rows whose scores take a launch of their own (over 640
+    tokens, in the scratch), and rows beyond the 18,432-token window."""
+    _check(torch_cuda, Oracle(), 100 + length, length, HEADS, KV_HEADS)
+
+
+@pytest.mark.parametrize("group", [1, 2, 4, 5, 6, 7, 8])
+def test_row_kernel_groups(torch_cuda, group):
+    """Every number of query heads per KV head, scores in the row kernel and
+    in the scratch."""
+    for length in (77, 1500):
+        _check(torch_cuda, Oracle(), 200 + group, length, 2 * group, 2)
+
+
+@pytest.mark.parametrize("scale,equal", [(0.0, False), (1.0, True), (8.0, False), (0.05, False)])
+def test_row_kernel_denominators(torch_cuda, scale, equal):
+    """Denominators that are exact in every step (equal scores: all e_t are
+    1, the sum crosses each power of two exactly), that hardly change after
+    a few tokens (peaked scores, many e_t far below one unit of the sum) and
+    that grow evenly."""
+    for length in (500, 5000):
+        _check(torch_cuda, Oracle(), 300, length, HEADS, KV_HEADS, scale, equal)
