@@ -111,6 +111,9 @@ __global__ __launch_bounds__(kWaves * 64, CH == 1 ? 4 : 1) void fast_gemm_kernel
     // barrier precedes the owners' sums; more tiles are summed in two levels
     // (wavefronts 4-7 into 0-3, then to the owners) to halve the LDS.
     constexpr bool kOneSync = T <= 4;
+    // Decode tiles (long chunks) stream their weights; launch_sized says why
+    // the others do not.
+    constexpr bool kStreamWeights = CH >= 6;
     __shared__ f4 part_s[kOneSync ? kWaves : kWaves / 2][T][64];
     __shared__ float ssq_s[NORM ? RB * 16 : 1][kSsqSlots];
     __shared__ float inv_s[RB * 16];
@@ -219,8 +222,10 @@ __global__ __launch_bounds__(kWaves * 64, CH == 1 ? 4 : 1) void fast_gemm_kernel
 #pragma unroll
                 for (int rb = 0; rb < RB; ++rb) av[c][rb] = ld4(xa[rb] + s * 1024);  // 4 quads x 64 rows x 4
 #pragma unroll
-                for (int j = 0; j < NB; ++j)
-                    bv[c][j] = __builtin_nontemporal_load(reinterpret_cast<const f4*>(wb[j] + s * 256));
+                for (int j = 0; j < NB; ++j) {
+                    const f4* w4 = reinterpret_cast<const f4*>(wb[j] + s * 256);
+                    bv[c][j] = kStreamWeights ? __builtin_nontemporal_load(w4) : *w4;
+                }
             }
         }
     };
@@ -243,27 +248,10 @@ __global__ __launch_bounds__(kWaves * 64, CH == 1 ? 4 : 1) void fast_gemm_kernel
             }
         }
     };
-    if constexpr (CH == 2) {
-        // Short chunks (the many-step tiles of the LM head and of prefill):
-        // two operand buffers, the next chunk's loads in flight during this
-        // chunk's MFMAs.
-        f4 av0[CH][RB], bv0[CH][NB], gv0[CH], av1[CH][RB], bv1[CH][NB], gv1[CH];
-        load(0, av0, bv0, gv0);
-        for (int i0 = 0; i0 < mine; i0 += 2 * CH) {
-            if (i0 + CH < mine) load(i0 + CH, av1, bv1, gv1);
-            __builtin_amdgcn_sched_barrier(0);
-            multiply(i0, av0, bv0, gv0);
-            if (i0 + CH >= mine) break;
-            if (i0 + 2 * CH < mine) load(i0 + 2 * CH, av0, bv0, gv0);
-            __builtin_amdgcn_sched_barrier(0);
-            multiply(i0 + CH, av1, bv1, gv1);
-        }
-    } else {
-        for (int i0 = 0; i0 < mine; i0 += CH) {
-            f4 av[CH][RB], bv[CH][NB], gv[CH];
-            load(i0, av, bv, gv);
-            multiply(i0, av, bv, gv);
-        }
+    for (int i0 = 0; i0 < mine; i0 += CH) {
+        f4 av[CH][RB], bv[CH][NB], gv[CH];
+        load(i0, av, bv, gv);
+        multiply(i0, av, bv, gv);
     }
     if (NORM) {
         float ss = 0.0f;
@@ -678,23 +666,30 @@ hipError_t launch_fast(hipStream_t s, const FastGemmArgs& a) {
 // Tile shape by size. At decode sizes (one row tile) the tiles are small,
 // for many work-groups (SwiGLU over more than 32 rows takes two row blocks:
 // its two weight matrices make its column blocks the heaviest; up to 32 rows one,
-// 6.3-6.5 instead of 8.0-8.7 us at 1 and 32 rows), and so up to 256 rows
-// (at 256 rows they beat the larger tiles below: O 6.6 vs 7.5, down 12.5 vs
-// 14.8, gate/up 16.9 vs 18.9 us). The LM head takes tiles of 64 columns
-// and 16, 32 or 64 rows, and a projection of more than 256 rows takes
-// 64 x 64 tiles when they still
-// give every CU a work-group: they read each weight and each activation a
-// quarter as often. Otherwise the largest of 64 x 16, 32 x 16 and 16 x 16
-// that gives every CU a work-group. (The q|k|v+RoPE projection keeps
-// 64 x 16 or 32 x 16 tiles above 64 rows, 11.2 vs 16.0 us at 256 rows, up to
-// where 64 x 64 tiles give every CU a work-group.)
+// 6.3-6.5 instead of 8.0-8.7 us at 1 and 32 rows). With many rows a tile of
+// 64 rows and 32 columns (two column blocks, of SwiGLU both matrices), or of
+// 64 x 16 where those are too few, reads weights and activations less often.
+// Either is taken from 7 work-groups per 4 CUs on: below, the wider tile
+// leaves CUs idle (SwiGLU of 512 rows, 384 tiles of 64 x 32: 28.5 vs 24.0 us
+// for 64 x 16; down at 512 rows, 288 of 64 x 16: 21.9 vs 20.0 for 16 x 16).
+// Such tiles take their steps one at a time (CH = 1): what hides their loads
+// is a second and third work-group on the CU, which the registers of longer
+// chunks kept out. us at 4,096 rows with CH = 2 and 64 x 64 before: gate/up
+// 189 -> 155, q|k|v 80 -> 68, O and down 186 -> 158 together; at 512 rows 31
+// -> 24, 16 -> 12.6, 43 -> 30; at 256 rows gate/up (two row blocks, CH = 3
+// instead of 6) 19.4 -> 17.0 and q|k|v 11.6 -> 8.9. From 65 rows on the weights
+// are read with plain loads: nontemporal ones made each row group fetch them
+// again past the L2 (gate/up 50 vs 47 us at 1,000 rows, 20.0 vs 18.4 at 256).
+// Decode tiles keep them (64 rows: q|k|v 6.3 vs 6.9 us, a whole step of the
+// 30-layer model 1.0% less).
 constexpr int kCus = 256;
 bool head_wide(int columns) { return columns % 64 == 0; }
 int tiles(const FastGemmArgs& a, int rb, int cb) { return ((a.rows + 15) / 16 + rb - 1) / rb * (a.columns / 16 / cb); }
 
+bool many(int tiles) { return 4 * tiles >= 7 * kCus; }
+
 template <int EPI, bool NORM, bool GATHER>
 hipError_t launch_sized(hipStream_t s, const FastGemmArgs& a) {
-    constexpr int M = EPI == kSwiglu ? 2 : 1;
     if constexpr (EPI == kHead) {
         if (a.inner == 576 && a.ssq_parts == 576 / 16 && head_wide(a.columns) && a.norm && a.ssq_in) {
             const int blocks = (a.columns / 16 + kHeadWaves - 1) / kHeadWaves;
@@ -712,14 +707,15 @@ hipError_t launch_sized(hipStream_t s, const FastGemmArgs& a) {
         }
         return launch_fast<EPI, NORM, GATHER, 1, 1, 6>(s, a);
     } else {
-        if (a.rows > 256) {
-            if (a.columns % 64 == 0 && tiles(a, 4, 4 / M) >= kCus)
-                return launch_fast<EPI, NORM, GATHER, 4, 4 / M, 2>(s, a);
-            if (tiles(a, 4, 1) >= kCus) return launch_fast<EPI, NORM, GATHER, 4, 1, 2>(s, a);
-            if (tiles(a, 2, 1) >= kCus) return launch_fast<EPI, NORM, GATHER, 2, 1, 6>(s, a);
-        }
-        if constexpr (M == 2) {
+        if (a.columns % 32 == 0 && many(tiles(a, 4, 2))) return launch_fast<EPI, NORM, GATHER, 4, 2, 1>(s, a);
+        if (many(tiles(a, 4, 1))) return launch_fast<EPI, NORM, GATHER, 4, 1, 1>(s, a);
+        if constexpr (EPI == kSwiglu) {
+            if (a.rows > 64) return launch_fast<EPI, NORM, GATHER, 2, 1, 3>(s, a);
             if (a.rows > 32) return launch_fast<EPI, NORM, GATHER, 2, 1, 6>(s, a);
+        } else if constexpr (EPI == kRope) {
+            if (a.rows > 64 && tiles(a, 2, 1) >= kCus) return launch_fast<EPI, NORM, GATHER, 2, 1, 3>(s, a);
+        } else {
+            if (a.rows > 256) return launch_fast<EPI, NORM, GATHER, 1, 1, 3>(s, a);
         }
         return launch_fast<EPI, NORM, GATHER, 1, 1, 12>(s, a);
     }
@@ -748,10 +744,7 @@ hipError_t launch_fast_gemm(hipStream_t s, Epilogue epilogue, const FastGemmArgs
         if (a.columns % kRopeDim || a.heads * kRopeDim + 2 * a.kv.kv_width != a.columns || !norm ||
             a.kv.block_tokens <= 0 || !a.row_block || !a.row_rope)
             return hipErrorInvalidValue;
-        if (a.rows > 256 && tiles(a, 4, 4) >= kCus) return launch_fast<kRope, true, false, 4, 4, 2>(s, a);
-        if (a.rows > 64 && tiles(a, 4, 1) >= kCus) return launch_fast<kRope, true, false, 4, 1, 2>(s, a);
-        if (a.rows > 64 && tiles(a, 2, 1) >= kCus) return launch_fast<kRope, true, false, 2, 1, 6>(s, a);
-        return launch_fast<kRope, true, false, 1, 1, 12>(s, a);
+        return launch_sized<kRope, true, false>(s, a);
     }
     return hipErrorInvalidValue;
 }
