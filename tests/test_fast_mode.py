@@ -348,6 +348,37 @@ def test_fast_prefill_rows_same_in_small_and_large_launches(torch_cuda, group):
     assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
 
 
+@pytest.mark.parametrize("count,vocabulary", [(17, 4096), (33, 192), (65, 4096), (129, 4096), (200, 64), (70, 12352)])
+def test_fast_head_rows_do_not_depend_on_the_passes(torch_cuda, count, vocabulary):
+    """The LM head deals its passes of 16, 32 or 64 rows over work-groups by
+    the rows and columns of the step: the logits and tokens of `count`
+    sequences decoded together equal those of the same sequences decoded in
+    groups of 16 (one pass each), bit for bit, and each row's token is its
+    own first maximum."""
+    cfg = smollm_config(layers=1, context=32, vocabulary=vocabulary)
+    model = OracleModel(cfg, seed=73)
+    o = Oracle()
+    tokens = [int(t) for t in o.fill_tokens(count, 73, 9800, vocabulary)]
+
+    def run(size):
+        backend = HipBackend(cfg, block_tokens=16, max_blocks=count, max_sequences=count, arithmetic=ARITHMETIC_FAST)
+        upload_model(backend, model)
+        for i in range(count):
+            backend.table_write(i, 0, np.array([i], dtype=np.int32))
+        out = []
+        for at in range(0, count, size):
+            group = range(at, min(at + size, count))
+            am, got = backend.forward([(i, 0, 2) for i in group], [t for i in group for t in (tokens[i], 1)])
+            for a, g in zip(am, got):
+                assert a == int(np.argmax(g))
+                out.append(g.copy())
+        backend.close()
+        return np.stack(out)
+
+    together, apart = run(count), run(16)
+    assert np.array_equal(together.view(np.uint32), apart.view(np.uint32))
+
+
 def test_fast_small_batch_decode_gemv(torch_cuda):
     """Decode steps of up to four sequences take the GEMV projections
     (row-major weights, RMSNorm computed inside the projections): 90

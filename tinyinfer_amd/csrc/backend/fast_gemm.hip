@@ -48,6 +48,7 @@
 // RMSNorm on the input (NORM): a[r][k] = x[r][k] * g[k], and the result is
 // scaled by 1/sqrt(sum_k x[r][k]^2 / K + eps), the sum assembled from the
 // producer's per-block partials.
+#include <algorithm>
 #include <type_traits>
 
 #include "kernels.h"
@@ -463,8 +464,9 @@ __global__ __launch_bounds__(kWaves * 64, CH == 1 ? 4 : 1) void fast_gemm_kernel
 // per output over the 16-k steps in order, the row blocks' MFMAs of a
 // sub-step issued together (41.7 us at 64 rows, 20.5 us at 16, measured in
 // isolation). The order depends on K only, so a row's logits do not depend
-// on the batch or on the rows sharing its pass; rows beyond 64 take further
-// passes over the same columns. Epilogue as above: the row's 1/sqrt(mean
+// on the batch or on the rows sharing its pass. Rows beyond a pass take
+// further passes over the same columns, in work-groups of their own (grid y)
+// where the columns leave CUs idle. Epilogue as above: the row's 1/sqrt(mean
 // square + eps) (its per-16-column partials summed in a fixed order), logits
 // on request, and per row and 64-column group the first maximum and a
 // non-finite flag, the four wavefronts of a group combined through LDS.
@@ -492,7 +494,8 @@ __global__ __launch_bounds__(kHeadWaves * 64, 1) void fast_head_kernel(FastGemmA
     const bool active = cb < nblocks;
     // Lane l's float4 of fragment (cb, s): W[16cb + l%16][16s + 4(l/16) .. +3].
     const float* wb = a.w + (size_t)min(cb, nblocks - 1) * S * 256 + (size_t)lane * 4;
-    for (int r0 = 0; r0 < a.rows; r0 += R) {
+    const int first = blockIdx.y * R;
+    for (int r0 = first; r0 < a.rows; r0 += gridDim.y * R) {
         // The thread index, opaque to the compiler in each pass: otherwise
         // it keeps every fill address live across the passes (spilled).
         int tid = threadIdx.x;
@@ -509,7 +512,7 @@ __global__ __launch_bounds__(kHeadWaves * 64, 1) void fast_head_kernel(FastGemmA
             const int xrow = a.row_map ? a.row_map[r] : r;
             xv[u] = ld4(a.x + ((size_t)(xrow >> 6) * (K / 4) * 64 + (xrow & 63)) * 4 + (size_t)(4 * s + (l >> 4)) * 256);
         }
-        if (r0 == 0 && tid < S * 4) gv = ld4(a.norm + 4 * tid);
+        if (r0 == first && tid < S * 4) gv = ld4(a.norm + 4 * tid);
         // The row's S per-16-column sums of squares: quarter q (partials
         // qS/4 .. (q+1)S/4 - 1, in order) by thread qR + row.
         float ss = 0.0f;
@@ -527,7 +530,7 @@ __global__ __launch_bounds__(kHeadWaves * 64, 1) void fast_head_kernel(FastGemmA
 #pragma unroll
         for (int j = 0; j < kHeadRing; ++j)
             ring[j] = __builtin_nontemporal_load(reinterpret_cast<const f4*>(wb + (size_t)j * 256));
-        if (r0 == 0 && tid < S * 4) g_s[tid / 4][tid % 4] = gv;
+        if (r0 == first && tid < S * 4) g_s[tid / 4][tid % 4] = gv;
         if (tid < 4 * R) ssq_s[tid / R][tid % R] = ss;
         __syncthreads();
         // The rows times the RMSNorm weights (so that the MFMA loop has no
@@ -693,9 +696,21 @@ hipError_t launch_sized(hipStream_t s, const FastGemmArgs& a) {
     if constexpr (EPI == kHead) {
         if (a.inner == 576 && a.ssq_parts == 576 / 16 && head_wide(a.columns) && a.norm && a.ssq_in) {
             const int blocks = (a.columns / 16 + kHeadWaves - 1) / kHeadWaves;
-            if (a.rows <= 16) fast_head_kernel<576, 1><<<blocks, kHeadWaves * 64, 0, s>>>(a);
-            else if (a.rows <= 32) fast_head_kernel<576, 2><<<blocks, kHeadWaves * 64, 0, s>>>(a);
-            else fast_head_kernel<576, 4><<<blocks, kHeadWaves * 64, 0, s>>>(a);
+            // Rows per pass: the fewest (16, 32 or 64) with which every pass
+            // over every run of columns has a CU of its own, 64 where none
+            // has. The whole vocabulary (49,152 columns, 256 runs) takes one
+            // pass of up to 64 rows; 4,096 columns (22 runs) at 256 rows take
+            // 8 passes of 32 side by side, 25.6 instead of 149 us for four
+            // passes one after the other, and at 64 rows four of 16, 16.4
+            // instead of 41 us.
+            auto passes = [&](int rb) { return (a.rows + 16 * rb - 1) / (16 * rb); };
+            const int rb = a.rows <= 16 || blocks * passes(1) <= kCus   ? 1
+                           : a.rows <= 32 || blocks * passes(2) <= kCus ? 2
+                                                                        : 4;
+            const dim3 grid(blocks, std::max(1, std::min(passes(rb), kCus / blocks)));
+            if (rb == 1) fast_head_kernel<576, 1><<<grid, kHeadWaves * 64, 0, s>>>(a);
+            else if (rb == 2) fast_head_kernel<576, 2><<<grid, kHeadWaves * 64, 0, s>>>(a);
+            else fast_head_kernel<576, 4><<<grid, kHeadWaves * 64, 0, s>>>(a);
             return hipGetLastError();
         }
         if (head_wide(a.columns)) {
