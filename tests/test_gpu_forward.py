@@ -120,6 +120,25 @@ def test_narrow_shape_short_weight_columns(torch_cuda):
     _run_sequence(model, backend, 16, chunks, table)
 
 
+@pytest.mark.parametrize("hidden,intermediate,vocabulary,rows", [(64, 192, 1000, 65), (128, 64, 52, 130),
+                                                                 (192, 100, 72, 70), (640, 704, 136, 129)])
+def test_prefill_projection_shapes(torch_cuda, hidden, intermediate, vocabulary, rows):
+    """Chunks of more than one row tile in the exact arithmetic: projections
+    of 1 to 11 whole 64-wide chunks of inner size (fewer and more than the
+    stages of the ring) and one that is not (100), columns that leave the
+    last work-group partly empty (8 columns each, 16 in the head), ragged
+    last row tiles, and the decode step after them, bit for bit."""
+    cfg = tiny_config(hidden=hidden, intermediate=intermediate, heads=hidden // 16, kv_heads=hidden // 32,
+                      vocabulary=vocabulary, context=192, tied=1)
+    model = OracleModel(cfg, seed=31, stddev=0.05)
+    backend = HipBackend(cfg, block_tokens=16, max_blocks=16, max_sequences=2)
+    upload_model(backend, model)
+    o = Oracle()
+    prompt = [int(t) for t in o.fill_tokens(rows + 3, 31, 3300, vocabulary)]
+    table = o.permutation(16, 31, 3301)[:12].copy()
+    _run_sequence(model, backend, 16, [prompt[:3], prompt[3:], prompt[:1]], table)
+
+
 def test_batched_rows_match_single_sequences(torch_cuda):
     """Several sequences in one forward call == each appended alone."""
     cfg = smollm_config(layers=2, context=256)

@@ -15,7 +15,9 @@
 // staging), NS-2 chunks ahead of the arithmetic. Each stage is a separate LDS
 // object so that the compiler's own LDS-DMA wait tracking tells stages
 // apart; the cross-wavefront hand-off is an explicit vmcnt wait plus a bare
-// s_barrier. Prefill and the LM head use this kernel with C > 1.
+// s_barrier. This kernel serves the shapes whose inner size is not a multiple
+// of 64; with whole 64-wide chunks, gemm_scalar_kernel (several row tiles and
+// the LM head) and the column kernels (decode) below do.
 //
 // Decode (one row tile) has too few outputs for C > 1, and with C = 1 the
 // LDS copy of the weights costs as much LDS bandwidth as x. There
@@ -77,8 +79,53 @@ __device__ __forceinline__ void bare_barrier() {
     asm volatile("" ::: "memory");
 }
 
-// FULL: inner % 64 == 0 and columns % kCols == 0 (no clamping anywhere).
-template <int C, int NW, int EPI, int NS, bool FULL>
+// Head epilogue of a work-group of NW wavefronts, lane = row, C columns n0..
+// of each wavefront in `acc`: the logits row-major on request, and per row the
+// first maximum over this lane's columns (std::max_element keeps the earliest
+// of equal values), then over the work-group's wavefronts in column order; one
+// partial per (row, work-group). Every wavefront calls it.
+template <int C, int NW>
+__device__ __forceinline__ void head_partials(const GemmArgs& a, const float (&acc)[C], int n0, int row) {
+    __shared__ float red_v[NW][64];
+    __shared__ int32_t red_i[NW][64];
+    __shared__ int32_t red_bad[NW][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const bool row_ok = row < a.rows;
+    float best = 0.0f;
+    int32_t best_i = -1, bad = 0;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int n = n0 + c;
+        if (n >= a.columns) break;
+        const float v = acc[c];
+        if (!isfinite(v)) bad = 1;
+        if (best_i < 0 || best < v) {
+            best = v;
+            best_i = n;
+        }
+        if (a.out && row_ok) a.out[(size_t)row * a.columns + n] = v;
+    }
+    red_v[wave][lane] = best;
+    red_i[wave][lane] = best_i;
+    red_bad[wave][lane] = bad;
+    __syncthreads();
+    if (wave == 0 && row_ok) {
+        for (int w = 1; w < NW; ++w) {
+            const int32_t i = red_i[w][lane];
+            if (i >= 0 && (best_i < 0 || best < red_v[w][lane])) {
+                best = red_v[w][lane];
+                best_i = i;
+            }
+            bad |= red_bad[w][lane];
+        }
+        const size_t p = (size_t)row * a.groups + blockIdx.x;
+        a.best_value[p] = best;
+        a.best_index[p] = best_i;
+        a.bad[p] = bad;
+    }
+}
+
+template <int C, int NW, int EPI, int NS>
 __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(GemmArgs a) {
     using S = Shape<C, NW, EPI>;
     constexpr int M = S::kMats;
@@ -116,7 +163,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(GemmArgs a) {
 #pragma unroll
         for (int j = 0; j < S::kXDma; ++j) {
             const int q = wave * S::kXDma + j;
-            const bool in = FULL || q0 + q < kq_total;
+            const bool in = q0 + q < kq_total;
             dma16(xsrc + (in ? (size_t)(q0 + q) * 64 + lane : 0), st.x + q * 64);
         }
 #pragma unroll
@@ -126,7 +173,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(GemmArgs a) {
                 const int cm = e / kQuads, q = e % kQuads;
                 const int c_ = cm / M, m = cm % M;
                 const int n = col0 + c_;
-                const bool in = FULL || (n < N && q0 + q < kq_total);
+                const bool in = n < N && q0 + q < kq_total;
                 const float4* src = (M == 2 && m) ? u4 : w4;
                 dma16(src + (in ? (size_t)n * kq_total + q0 + q : 0), st.w + wave * S::kWaveW4 + j * 64);
             }
@@ -175,7 +222,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(GemmArgs a) {
     // arithmetic; with C chains per lane a quad's own reads are enough.
     constexpr int kDepth = 4;
     auto compute = [&](const St& st, int nq) {
-        if (C == 1 && (FULL || nq == kQuads)) {
+        if (C == 1 && nq == kQuads) {
             float4 xv[kDepth];
             float4 wv[kDepth][M][C];
 #pragma unroll
@@ -229,51 +276,17 @@ __global__ __launch_bounds__(NW * 64) void gemm_rows_kernel(GemmArgs a) {
     const int row = tile * 64 + lane;
     const bool row_ok = row < a.rows;
     if (EPI == kHead) {
-        // First maximum over this lane's columns (std::max_element keeps the
-        // earliest of equal values), then over the work-group's wavefronts
-        // in column order; one partial per (row, work-group).
-        __shared__ float red_v[NW][64];
-        __shared__ int32_t red_i[NW][64];
-        __shared__ int32_t red_bad[NW][64];
-        float best = 0.0f;
-        int32_t best_i = -1, bad = 0;
+        float v[C];
 #pragma unroll
-        for (int c = 0; c < C; ++c) {
-            const int n = n0 + wave * C + c;
-            if (!FULL && n >= N) break;
-            const float v = acc[0][c];
-            if (!isfinite(v)) bad = 1;
-            if (best_i < 0 || best < v) {
-                best = v;
-                best_i = n;
-            }
-            if (a.out && row_ok) a.out[(size_t)row * N + n] = v;
-        }
-        red_v[wave][lane] = best;
-        red_i[wave][lane] = best_i;
-        red_bad[wave][lane] = bad;
-        __syncthreads();
-        if (wave == 0 && row_ok) {
-            for (int w = 1; w < NW; ++w) {
-                const int32_t i = red_i[w][lane];
-                if (i >= 0 && (best_i < 0 || best < red_v[w][lane])) {
-                    best = red_v[w][lane];
-                    best_i = i;
-                }
-                bad |= red_bad[w][lane];
-            }
-            const size_t p = (size_t)row * a.groups + blockIdx.x;
-            a.best_value[p] = best;
-            a.best_index[p] = best_i;
-            a.bad[p] = bad;
-        }
+        for (int c = 0; c < C; ++c) v[c] = acc[0][c];
+        head_partials<C, NW>(a, v, n0 + wave * C, row);
         return;
     }
     if (!row_ok) return;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
         const int n = n0 + wave * C + c;
-        if (!FULL && n >= N) break;
+        if (n >= N) break;
         float* o = a.out + quad_index(row, n, N);
         if (EPI == kStore) {
             *o = acc[0][c];
@@ -337,14 +350,202 @@ template <int C, int NW, int EPI, int NS>
 hipError_t launch_shape(hipStream_t s, const GemmArgs& a) {
     using S = Shape<C, NW, EPI>;
     const dim3 grid((a.columns + S::kCols - 1) / S::kCols, (a.rows + 63) / 64);
-    const bool full = a.inner % kChunk == 0 && a.columns % S::kCols == 0;
-    if (full)
-        gemm_rows_kernel<C, NW, EPI, NS, true><<<grid, S::kThreads, 0, s>>>(a);
-    else
-        gemm_rows_kernel<C, NW, EPI, NS, false><<<grid, S::kThreads, 0, s>>>(a);
+    gemm_rows_kernel<C, NW, EPI, NS><<<grid, S::kThreads, 0, s>>>(a);
     return hipGetLastError();
 }
 
+
+// ---------------------------------------------------------------------------
+// Projections of several row tiles, inner a multiple of 64: C columns per
+// wavefront as above, but the weights come as scalar operands. A column's
+// weights are the same for every lane, so a wavefront reads them with scalar
+// loads (W consecutive k of each of its columns, the next ones in flight) and
+// each product is one v_mul_f32 with a scalar operand. gemm_rows_kernel reads
+// them as LDS broadcasts, which cost the LDS as much as the x quads do: with
+// C = 4 five 1 KB reads per quad and wavefront, 160 LDS cycles for the CU's
+// four against 152 of arithmetic; here LDS serves x only. What bounds it then
+// is the VALU: two instructions per product and sum (multiply and add are
+// rounded separately), 4 cycles each.
+// us at 256 rows before and now: gate/up 71 -> 28, down 50 -> 22 (31.7 without the
+// lines touched first), q|k|v 21.6 -> 10.8, O 20 -> 11; at 1,000 rows gate/up takes
+// 92 (the VALU 90); the head of 64 rows 35 -> 11.8 over 4,096 columns, 127 -> 95
+// over 49,152 (the VALU 92).
+// Columns per wavefront: with two a run is 16 k (64 scalar registers for this
+// run's weights and the next one's), whose arithmetic covers a scalar load
+// even where a SIMD has one wavefront; 3 and 4 columns of 8 k took 40.7 us for
+// down.
+constexpr int kScalarColumns = 2;
+constexpr int kScalarStages = 3;  // three work-groups per CU (four stages, two: gate/up 38.6 us)
+
+typedef const __attribute__((address_space(4))) float* ScalarPtr;
+template <int W>
+struct ScalarRun {
+    typedef float type __attribute__((ext_vector_type(W)));
+};
+
+template <int NW, int EPI>
+__global__ __launch_bounds__(NW * 64) void gemm_scalar_kernel(GemmArgs a) {
+    constexpr int C = kScalarColumns, M = EPI == kSwiglu ? 2 : 1;
+    constexpr int CM = C * M;
+    constexpr int W = 32 / CM;  // two runs of every column fill 64 scalar registers
+    constexpr int NS = kScalarStages;
+    constexpr int D = kQuads / NW;  // 1 KB copies per wavefront and chunk
+    typedef typename ScalarRun<W>::type Run;
+    typedef const __attribute__((address_space(4))) Run* RunPtr;
+    using St = Stage<64 * kQuads, 1>;
+    __shared__ St st0, st1, st2;
+    __shared__ float touched[64];  // never read
+    auto stage = [&](int s) -> St& {
+        switch (s) {
+        case 0: return st0;
+        case 1: return st1;
+        default: return st2;
+        }
+    };
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tile = blockIdx.y;
+    const int n0 = (blockIdx.x * NW + wave) * C;
+    const int K = a.inner, N = a.columns, chunks = K / kChunk;
+    const float4* xsrc = reinterpret_cast<const float4*>(a.x) + (size_t)tile * (K >> 2) * 64;
+    ScalarPtr w[CM];
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+            w[c * M + m] = (ScalarPtr)((m ? a.w2 : a.w) + (size_t)min(n0 + c, N - 1) * K);
+    auto issue = [&](int c, St& st) {
+#pragma unroll
+        for (int j = 0; j < D; ++j) {
+            const int q = wave * D + j;
+            dma16(xsrc + (size_t)(c * kQuads + q) * 64 + lane, st.x + q * 64);
+        }
+    };
+    auto wait_chunks = [&](int later) {
+        switch (later) {
+        case 0: wait_vm<0>(); break;
+        case 1: wait_vm<D>(); break;
+        default: wait_vm<(NS - 2) * D>(); break;
+        }
+    };
+    // One dword of every 128-byte line of this wavefront's weights: a scalar
+    // load that finds its line in the L2 comes back within a run.
+    {
+        const int lines = K >> 5;
+        for (int i = lane; i < CM * lines; i += 64) {
+            const int c = i / lines;
+            const float* src = (M == 2 && c % M ? a.w2 : a.w) + (size_t)min(n0 + c / M, N - 1) * K + 32 * (i - c * lines);
+            __builtin_amdgcn_global_load_lds((const void*)src, (LdsPtr)touched, 4, 0, 0);
+        }
+    }
+    float acc[CM];
+    Run wn[CM];
+#pragma unroll
+    for (int c = 0; c < CM; ++c) {
+        acc[c] = 0.0f;
+        wn[c] = *(RunPtr)w[c];
+    }
+    // Chunk c: runs of W k, the weights of the next run (the next chunk's
+    // first at the end) and the x quads of the next one read during this.
+    auto compute = [&](const St& st, int c) {
+        constexpr int Q = W / 4, R = kChunk / W;
+        float4 xn[Q];
+#pragma unroll
+        for (int j = 0; j < Q; ++j) xn[j] = st.x[j * 64 + lane];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            float4 x[Q];
+            Run wv[CM];
+#pragma unroll
+            for (int j = 0; j < Q; ++j) x[j] = xn[j];
+#pragma unroll
+            for (int i = 0; i < CM; ++i) wv[i] = wn[i];
+            // This run's operands have arrived; only then the next run's are
+            // requested (scalar loads return in any order, so a later wait
+            // for these would wait for those too).
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt 0
+            __builtin_amdgcn_sched_barrier(0);
+            if (r + 1 < R)
+#pragma unroll
+                for (int j = 0; j < Q; ++j) xn[j] = st.x[((r + 1) * Q + j) * 64 + lane];
+            if (r + 1 == R) {
+                // The next chunk's first run (after the last chunk, the row's
+                // first again, unused).
+                const int next = c + 1 < chunks ? kChunk : kChunk - K;
+#pragma unroll
+                for (int i = 0; i < CM; ++i) w[i] += next;
+            }
+            // (The empty asm keeps the compiler from merging several runs'
+            // loads, which the scalar registers cannot hold.)
+#pragma unroll
+            for (int i = 0; i < CM; ++i) {
+                asm volatile("" : "+s"(w[i]));
+                wn[i] = *(RunPtr)(w[i] + (r + 1 == R ? 0 : (r + 1) * W));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < Q; ++j) {
+#pragma unroll
+                for (int i = 0; i < CM; ++i) acc[i] = acc[i] + x[j].x * wv[i][4 * j];
+#pragma unroll
+                for (int i = 0; i < CM; ++i) acc[i] = acc[i] + x[j].y * wv[i][4 * j + 1];
+#pragma unroll
+                for (int i = 0; i < CM; ++i) acc[i] = acc[i] + x[j].z * wv[i][4 * j + 2];
+#pragma unroll
+                for (int i = 0; i < CM; ++i) acc[i] = acc[i] + x[j].w * wv[i][4 * j + 3];
+            }
+            // The run's arithmetic stays before the next run's wait.
+#pragma unroll
+            for (int i = 0; i < CM; ++i) asm volatile("" : "+v"(acc[i]));
+        }
+    };
+    // The stage pipeline of gemm_rows_kernel.
+#pragma unroll
+    for (int s = 0; s < NS - 1; ++s)
+        if (s < chunks) issue(s, stage(s));
+    wait_chunks(min(NS - 2, chunks - 1));
+    bare_barrier();
+    for (int c0 = 0; c0 < chunks; c0 += NS) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            const int c = c0 + s;
+            if (c >= chunks) break;
+            compute(stage(s), c);
+            if (c + 1 < chunks) {
+                wait_chunks(min(c + NS - 2, chunks - 1) - (c + 1));
+                bare_barrier();
+                if (c + NS - 1 < chunks) issue(c + NS - 1, stage((s + NS - 1) % NS));
+            }
+        }
+    }
+    const int row = tile * 64 + lane;
+    if constexpr (EPI == kHead) {
+        head_partials<C, NW>(a, acc, n0, row);
+        return;
+    }
+    if (row >= a.rows) return;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int n = n0 + c;
+        if (n >= N) break;
+        float* o = a.out + quad_index(row, n, N);
+        if (EPI == kStore) {
+            *o = acc[c];
+        } else if (EPI == kResidual) {
+            *o = *o + acc[c];
+        } else {
+            const float g = acc[c * M];
+            *o = (g / (1.0f + ref_expf(-g))) * acc[c * M + M - 1];
+        }
+    }
+}
+
+template <int NW, int EPI>
+hipError_t launch_scalar(hipStream_t s, const GemmArgs& a) {
+    constexpr int kCols = NW * kScalarColumns;
+    gemm_scalar_kernel<NW, EPI><<<dim3((a.columns + kCols - 1) / kCols, (a.rows + 63) / 64), NW * 64, 0, s>>>(a);
+    return hipGetLastError();
+}
 
 // ---------------------------------------------------------------------------
 // Decode projections: one output column per wavefront.
@@ -778,8 +979,17 @@ hipError_t launch_gemm(hipStream_t s, Epilogue epilogue, const GemmArgs& a) {
     if (a.rows <= 0 || a.columns <= 0) return hipSuccess;
     if (a.inner <= 0 || a.inner % 4 || a.columns % 4) return hipErrorInvalidValue;
     // One row tile (decode): one column per wavefront with register-held
-    // weights. More rows: C = 4 columns per wavefront through LDS.
+    // weights. More rows: several columns per wavefront, their weights as
+    // scalars (through LDS where a row of weights is not a multiple of 64).
     const bool many = a.rows > 64;
+    if (many && a.inner % kChunk == 0) {
+        switch (epilogue) {
+        case kStore: return launch_scalar<4, kStore>(s, a);
+        case kResidual: return launch_scalar<4, kResidual>(s, a);
+        case kSwiglu: return launch_scalar<4, kSwiglu>(s, a);
+        default: break;
+        }
+    }
     if (!many && a.inner % 64 == 0) {
         switch (epilogue) {
         case kStore: return launch_column_one<kStore>(s, a);
@@ -794,11 +1004,10 @@ hipError_t launch_gemm(hipStream_t s, Epilogue epilogue, const GemmArgs& a) {
     case kStore: return many ? launch_shape<4, 4, kStore, 5>(s, a) : launch_shape<1, 4, kStore, 6>(s, a);
     case kResidual: return many ? launch_shape<4, 4, kResidual, 5>(s, a) : launch_shape<1, 4, kResidual, 6>(s, a);
     case kSwiglu: return many ? launch_shape<4, 4, kSwiglu, 5>(s, a) : launch_shape<1, 4, kSwiglu, 6>(s, a);
-    case kHead: {
-        using S = Shape<kHeadColumns / 8, 8, kHead>;
-        static_assert(S::kCols == kHeadColumns, "head work-group width");
-        return launch_shape<kHeadColumns / 8, 8, kHead, 4>(s, a);
-    }
+    case kHead:
+        static_assert(8 * kScalarColumns == kHeadColumns, "head work-group width");
+        if (a.inner % kChunk == 0) return launch_scalar<8, kHead>(s, a);
+        return launch_shape<kScalarColumns, 8, kHead, 4>(s, a);
     }
     return hipErrorInvalidValue;
 }

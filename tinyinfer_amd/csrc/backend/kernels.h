@@ -54,7 +54,7 @@ struct GemmArgs {
     int32_t* bad;
     int groups;
 };
-constexpr int kHeadColumns = 64;
+constexpr int kHeadColumns = 16;
 int head_groups(int columns);
 hipError_t launch_gemm(hipStream_t s, Epilogue epilogue, const GemmArgs& args);
 // The same projection of RMSNorm(x) (llama_runner.cpp:10-16 then :30-36)
