@@ -188,3 +188,59 @@ def test_fast_attention_rejects_other_shapes(torch_cuda):
                                                           1, 0, 1, bt, heads, kvh, dim, p, None)
         assert status == -1, (bt, heads, kvh, dim, length)
         assert lib().mp_hip_last_error(None)
+
+
+def test_fast_attention_calls_share_their_work_memory(torch_cuda):
+    """Calls take their work lists and partials from sets that earlier calls
+    left: calls of other sizes in between, eight threads at once on streams
+    of their own (more than the sets kept), and the destruction of a context
+    (which gives idle sets back) leave every result as the first call gave
+    it, bit for bit. Rows of 5 and 200 tokens (page ids filled in on the
+    device), 700 and 5,000 (splits)."""
+    import threading
+    from concurrent.futures import ThreadPoolExecutor
+
+    from tinyinfer_amd.backend import HipBackend
+    from .helpers import tiny_config
+    torch = torch_cuda
+    o = Oracle()
+    sets = []
+    for i, lengths in enumerate(([5, 200, 700, 5000], [17], [3000] * 40, [256, 1, 257])):
+        pages = [(n + 15) // 16 for n in lengths]
+        blocks = sum(pages)
+        dev = lambda n, stream, std=1.0: torch.from_numpy(o.fill_normal(n, 500 + i, stream, std)).cuda()
+        tables = torch.zeros((len(lengths), max(pages)), dtype=torch.int32)
+        perm, at = o.permutation(blocks, 500 + i, 9), 0
+        for row, p in zip(tables, pages):
+            row[:p] = torch.from_numpy(perm[at:at + p].copy())
+            at += p
+        sets.append((dev(len(lengths) * HEADS * DIM, 1), dev(blocks * BT * KVW, 2), dev(blocks * BT * KVW, 3),
+                     tables.cuda(), np.asarray(lengths, dtype=np.int32)))
+    torch.cuda.synchronize()
+
+    def call(which, stream):
+        q, k, v, t, lengths = sets[which]
+        with torch.cuda.stream(stream):
+            out = torch.full((len(lengths), HEADS * DIM), float("nan"), device="cuda")
+            paged_attention_decode_fast(q.data_ptr(), k.data_ptr(), v.data_ptr(), t.data_ptr(), t.shape[1], lengths, 0,
+                                        1, HEADS, KV_HEADS, out.data_ptr(), stream.cuda_stream)
+            stream.synchronize()
+        return out.cpu().numpy().view(np.uint32)
+
+    main = torch.cuda.current_stream()
+    first = [call(i, main) for i in range(4)]
+    for i in (2, 0, 3, 1, 0, 2):
+        assert np.array_equal(call(i, main), first[i]), i
+    start = threading.Barrier(8)
+
+    def worker(n):
+        torch.cuda.set_device(0)
+        stream = torch.cuda.Stream()
+        start.wait()
+        return all(np.array_equal(call((n + j) % 4, stream), first[(n + j) % 4]) for j in range(6))
+
+    with ThreadPoolExecutor(8) as pool:
+        assert all(pool.map(worker, range(8)))
+    HipBackend(tiny_config(), block_tokens=4, max_blocks=8, max_sequences=4).close()
+    for i in range(4):
+        assert np.array_equal(call(i, main), first[i]), i

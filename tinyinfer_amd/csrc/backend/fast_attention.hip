@@ -348,6 +348,16 @@ __global__ __launch_bounds__(kSplitPages * 64) void fast_attention_short_kernel(
     out[act_index<PLAIN>(row, (kvh * G + h) * kDim + lane, ldo)] = num / den;
 }
 
+__global__ __launch_bounds__(256) void short_pages_kernel(const int32_t* __restrict__ tables, int table_stride,
+                                                          int32_t* __restrict__ items, int count) {
+    constexpr int kIds = kShortItemInts - 4;
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= count * kIds) return;
+    int32_t* item = items + (size_t)(i / kIds) * kShortItemInts;
+    const int k = i % kIds, pages = (item[2] + kPage - 1) / kPage;
+    item[4 + k] = tables[(size_t)item[0] * table_stride + min(k, pages - 1)];
+}
+
 // out[row][h*64 + d] for the listed rows (w.merge_rows: one-token rows of
 // more than 256 tokens, with their sequences): the splits of (row, h/G)
 // combined. One wavefront
@@ -477,6 +487,12 @@ hipError_t launch_all(hipStream_t s, const float* qkv, int ldq, int heads, int k
 }
 
 }  // namespace
+
+hipError_t launch_short_pages(hipStream_t s, const int32_t* tables, int table_stride, int32_t* items, int count) {
+    if (count <= 0) return hipSuccess;
+    short_pages_kernel<<<(count * (kShortItemInts - 4) + 255) / 256, 256, 0, s>>>(tables, table_stride, items, count);
+    return hipGetLastError();
+}
 
 hipError_t launch_fast_attention(hipStream_t s, const float* qkv, int ldq, int rows, int heads, int kv_heads,
                                  const RowMeta& meta, const PagedKv& kv, int layer, float* out, int ldo,

@@ -250,6 +250,10 @@ struct FastAttentionWork {
 bool fast_prefill_fits(int heads, int kv_heads, const PagedKv& kv);
 hipError_t launch_fast_prefill(hipStream_t s, const float* qkv, int ldq, int heads, int kv_heads, const PagedKv& kv,
                                int layer, const int32_t* items, int count, float* out, int ldo);
+// The page ids (int32 4..19) of `count` short items, from row `item[0]`'s page
+// table at tables + row * table_stride (items of a caller whose tables the
+// host does not hold).
+hipError_t launch_short_pages(hipStream_t s, const int32_t* tables, int table_stride, int32_t* items, int count);
 // `plain`: q rows (ldq wide) and out rows (ldo wide) are row-major instead
 // of the quad layout (the stand-alone entry point).
 hipError_t launch_fast_attention(hipStream_t s, const float* qkv, int ldq, int rows, int heads, int kv_heads,
