@@ -190,6 +190,38 @@ def test_fast_attention_rejects_other_shapes(torch_cuda):
         assert lib().mp_hip_last_error(None)
 
 
+@pytest.mark.parametrize("group", [1, 2, 3, 4])
+def test_short_rows_same_alone_and_in_a_batch(torch_cuda, group):
+    """Rows of up to 256 tokens: few of them run each query head in a
+    work-group of its own, many a KV head's together. Rows of a batch of 140
+    (280 items, over 256 heads) equal the same rows called alone, bit for
+    bit, at lengths around the pages and splits."""
+    torch = torch_cuda
+    o = Oracle()
+    kv_heads, rows = 2, 140
+    edges = [1, 15, 16, 17, 128, 129, 144, 191, 255, 256]
+    lengths = np.asarray((edges + [int(x) for x in 1 + o.fill_tokens(rows, 91, 1, 256)])[:rows], dtype=np.int32)
+    blocks = 64
+    dev = lambda n, stream: torch.from_numpy(o.fill_normal(n, 91, stream, 1.0)).cuda()
+    q = dev(rows * kv_heads * group * DIM, 2)
+    k, v = dev(blocks * BT * kv_heads * DIM, 3), dev(blocks * BT * kv_heads * DIM, 4)
+    tables = torch.from_numpy(o.fill_tokens(rows * 16, 91, 5, blocks).astype(np.int32)).cuda()
+    width = kv_heads * group * DIM
+
+    def call(first, count):
+        out = torch.full((count, width), float("nan"), device="cuda")
+        paged_attention_decode_fast(q[first * width:].data_ptr(), k.data_ptr(), v.data_ptr(),
+                                    tables[first * 16:].data_ptr(), 16, lengths[first:first + count], 0, 1,
+                                    kv_heads * group, kv_heads, out.data_ptr(), None)
+        torch.cuda.synchronize()
+        return out.cpu().numpy()
+
+    together = call(0, rows)
+    assert np.all(np.isfinite(together))
+    for r in range(len(edges)):
+        assert np.array_equal(call(r, 1)[0].view(np.uint32), together[r].view(np.uint32)), int(lengths[r])
+
+
 def test_fast_attention_calls_share_their_work_memory(torch_cuda):
     """Calls take their work lists and partials from sets that earlier calls
     left: calls of other sizes in between, eight threads at once on streams

@@ -63,6 +63,13 @@ constexpr int kMaxPages = 16;    // pages of one split
 constexpr int kRing = 2;                           // pages in flight per wavefront
 constexpr int kItemsPerGroup = 4;
 constexpr int kMergeHeld = 16;  // splits per lane group whose partials the merge loads in one round
+// Query heads of short rows in work-groups of their own up to this many, one
+// per CU: a wavefront's chain over its pages is then one head's instead of G
+// heads', which is what a small batch waits for. Apart against together: 5.9
+// vs 8.2 us for one row of 191 tokens, 9.6 vs 11.0 for 16 rows (144 heads),
+// 11.0 vs 11.1 to 12.4 for 28 (252), but 16.1 vs 12.1 for 56 (504), where the
+// work-groups queue for CUs.
+constexpr int kShortApart = 256;
 constexpr float kScale = 0.125f;  // 1/sqrt(64)
 constexpr float kRescale = 16.0f;  // probabilities stay below e^16 before a rescale
 
@@ -88,7 +95,7 @@ __device__ __forceinline__ float touch_weights(const FastAttentionWork& w, uint6
 
 // One split: tokens t0..t0+n-1 (t0 page-aligned, at most kMaxPages pages)
 // of the row whose page ids are `table` (its page table, or the page ids a
-// short item carries), for the G query heads of KV head
+// short item carries), for G query heads from head0 on of KV head
 // kvh. Gives per head the reference maximum m, the denominator l and lane
 // d's weighted sum acc (not yet divided). `touch` numbers this wavefront's
 // 8 KB slice of the weight prefetch; p_s is the wavefront's own LDS.
@@ -100,7 +107,7 @@ __device__ __forceinline__ float touch_weights(const FastAttentionWork& w, uint6
 template <int G, bool PLAIN, int NP = 0>
 __device__ __forceinline__ void attend_split(const float* __restrict__ qkv, int ldq, const PagedKv& kv, int layer,
                                              const FastAttentionWork& w, const int32_t* table, int row, int kvh,
-                                             int t0, int n, uint64_t touch, float (&p_s)[G][kPage], float (&m)[G],
+                                             int head0, int t0, int n, uint64_t touch, float (&p_s)[G][kPage], float (&m)[G],
                                              float (&l)[G], float (&acc)[G]) {
     const int lane = threadIdx.x & 63;
     const int t = lane >> 2, dq = lane & 3;
@@ -131,7 +138,7 @@ __device__ __forceinline__ void attend_split(const float* __restrict__ qkv, int 
     for (int h = 0; h < G; ++h)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int c = (kvh * G + h) * kDim + dq * 16 + j * 4;
+            const int c = (head0 + h) * kDim + dq * 16 + j * 4;
             q[h][j] = *reinterpret_cast<const f4*>(qkv + act_index<PLAIN>(row, c, ldq));
         }
     __builtin_amdgcn_sched_barrier(0);
@@ -259,11 +266,11 @@ __global__ __launch_bounds__(kItemsPerGroup * 64) void fast_attention_kernel(con
     // variants that load exactly their pages.
     const int pages = __builtin_amdgcn_readfirstlane(n == 8 * kPage ? 8 : n == 16 * kPage ? 16 : 0);
     if (pages == 8)
-        attend_split<G, PLAIN, 8>(qkv, ldq, kv, layer, w, table, row, kvh, t0, n, (uint64_t)index, p_s[wave], m, l, acc);
+        attend_split<G, PLAIN, 8>(qkv, ldq, kv, layer, w, table, row, kvh, kvh * G, t0, n, (uint64_t)index, p_s[wave], m, l, acc);
     else if (pages == 16)
-        attend_split<G, PLAIN, 16>(qkv, ldq, kv, layer, w, table, row, kvh, t0, n, (uint64_t)index, p_s[wave], m, l, acc);
+        attend_split<G, PLAIN, 16>(qkv, ldq, kv, layer, w, table, row, kvh, kvh * G, t0, n, (uint64_t)index, p_s[wave], m, l, acc);
     else
-        attend_split<G, PLAIN>(qkv, ldq, kv, layer, w, table, row, kvh, t0, n, (uint64_t)index, p_s[wave], m, l, acc);
+        attend_split<G, PLAIN>(qkv, ldq, kv, layer, w, table, row, kvh, kvh * G, t0, n, (uint64_t)index, p_s[wave], m, l, acc);
     const size_t slot = ((size_t)seq * w.kv_heads + kvh) * w.split_stride + sp;
 #pragma unroll
     for (int h = 0; h < G; ++h) {
@@ -278,26 +285,30 @@ __global__ __launch_bounds__(kItemsPerGroup * 64) void fast_attention_kernel(con
 
 // Rows of up to 256 tokens (fast_attention_short: at most kSplitPages
 // splits of 16 or 32 tokens): one work-group per (row, KV head) of
-// w.short_items, wavefront s takes split s, and the splits are combined
+// w.short_items and run of HG of its G query heads, wavefront s takes split
+// s, and the splits are combined
 // through LDS in split order by one wavefront per query head, so these
-// rows need no merge launch. A row of one split gives acc / l exactly.
-template <int G, bool PLAIN>
+// rows need no merge launch. A row of one split gives acc / l exactly. A
+// head's result does not depend on HG.
+template <int G, bool PLAIN, int HG>
 __global__ __launch_bounds__(kSplitPages * 64) void fast_attention_short_kernel(const float* __restrict__ qkv,
                                                                                 int ldq, RowMeta meta, PagedKv kv,
                                                                                 int layer, FastAttentionWork w,
                                                                                 float* __restrict__ out, int ldo) {
+    static_assert(G % HG == 0, "equal runs of heads");
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    __shared__ float p_s[kSplitPages][G][kPage];
-    __shared__ float part_ml[kSplitPages][G][2];
-    __shared__ float part_acc[kSplitPages][G][kDim];
+    __shared__ float p_s[kSplitPages][HG][kPage];
+    __shared__ float part_ml[kSplitPages][HG][2];
+    __shared__ float part_acc[kSplitPages][HG][kDim];
+    const int index = (int)blockIdx.x / (G / HG), h0 = (int)blockIdx.x % (G / HG) * HG;
     // (row, slot * kv_heads + KV head, tokens, 0, page ids): the length and
     // the pages ride in the item, loaded together with the count, so the
     // pages' loads depend on one load only.
-    const int32_t* it = w.short_items + (size_t)min((int)blockIdx.x, w.short_capacity - 1) * kShortItemInts;
+    const int32_t* it = w.short_items + (size_t)min(index, w.short_capacity - 1) * kShortItemInts;
     int4 item = reinterpret_cast<const int4*>(it)[0];
-    if ((int)blockIdx.x >= w.short_capacity) item = {0, 0, 1, 0};
-    if ((int)blockIdx.x >= (w.counts ? w.counts[1] : w.short_count)) {
+    if (index >= w.short_capacity) item = {0, 0, 1, 0};
+    if (index >= (w.counts ? w.counts[1] : w.short_count)) {
         // A work-group past the items (small batches, whose items leave
         // most CUs idle) only touches its slices of the weights to prefetch.
         const float touched = touch_weights(w, (uint64_t)blockIdx.x * kSplitPages + wave, lane);
@@ -305,20 +316,21 @@ __global__ __launch_bounds__(kSplitPages * 64) void fast_attention_short_kernel(
         return;
     }
     const int row = item.x, kvh = item.y % w.kv_heads, length = item.z;
+    const int head0 = kvh * G + h0;
     const int32_t* table = it + 4;
     const int split = fast_attention_split(length);
     const int splits = (length + split - 1) / split;  // 1..kSplitPages
     if (wave < splits) {
-        float m[G], l[G], acc[G];
+        float m[HG], l[HG], acc[HG];
         const int t0 = wave * split;
         const int n = min(split, length - t0);
         const uint64_t touch = (uint64_t)blockIdx.x * kSplitPages + wave;
         if (n == 2 * kPage)  // whole 32-token splits: exactly their two pages
-            attend_split<G, PLAIN, 2>(qkv, ldq, kv, layer, w, table, row, kvh, t0, n, touch, p_s[wave], m, l, acc);
+            attend_split<HG, PLAIN, 2>(qkv, ldq, kv, layer, w, table, row, kvh, head0, t0, n, touch, p_s[wave], m, l, acc);
         else
-            attend_split<G, PLAIN>(qkv, ldq, kv, layer, w, table, row, kvh, t0, n, touch, p_s[wave], m, l, acc);
+            attend_split<HG, PLAIN>(qkv, ldq, kv, layer, w, table, row, kvh, head0, t0, n, touch, p_s[wave], m, l, acc);
 #pragma unroll
-        for (int h = 0; h < G; ++h) {
+        for (int h = 0; h < HG; ++h) {
             part_acc[wave][h][lane] = acc[h];
             if (lane == 0) {
                 part_ml[wave][h][0] = m[h];
@@ -327,7 +339,7 @@ __global__ __launch_bounds__(kSplitPages * 64) void fast_attention_short_kernel(
         }
     }
     __syncthreads();
-    if (wave >= G) return;
+    if (wave >= HG) return;
     // Query head h: lane s < splits holds split s's (maximum, denominator)
     // (all in the first 16-lane row), lane d sums its dimension over the
     // splits in order.
@@ -345,7 +357,7 @@ __global__ __launch_bounds__(kSplitPages * 64) void fast_attention_short_kernel(
 #pragma unroll
     for (int s = 0; s < kSplitPages; ++s)
         if (s < splits) num += part_acc[s][h][lane] * lane_value(f, s);
-    out[act_index<PLAIN>(row, (kvh * G + h) * kDim + lane, ldo)] = num / den;
+    out[act_index<PLAIN>(row, (head0 + h) * kDim + lane, ldo)] = num / den;
 }
 
 __global__ __launch_bounds__(256) void short_pages_kernel(const int32_t* __restrict__ tables, int table_stride,
@@ -458,10 +470,14 @@ void launch_items(hipStream_t s, const float* qkv, int ldq, const RowMeta& meta,
     if (shorts > 0) {
         // Without split items (whose launch covers the slices), enough
         // work-groups for every slice.
-        int groups = shorts;
+        const bool apart = shorts * G <= kShortApart;
+        int groups = apart ? shorts * G : shorts;
         if (items <= 0)
             groups = (int)std::max<uint64_t>((uint64_t)groups, (slices + kSplitPages - 1) / kSplitPages);
-        fast_attention_short_kernel<G, PLAIN><<<groups, kSplitPages * 64, 0, s>>>(qkv, ldq, meta, kv, layer, w, out, ldo);
+        if (apart)
+            fast_attention_short_kernel<G, PLAIN, 1><<<groups, kSplitPages * 64, 0, s>>>(qkv, ldq, meta, kv, layer, w, out, ldo);
+        else
+            fast_attention_short_kernel<G, PLAIN, G><<<groups, kSplitPages * 64, 0, s>>>(qkv, ldq, meta, kv, layer, w, out, ldo);
     }
     if (items > 0) {
         const uint64_t waves = std::max<uint64_t>((uint64_t)items, slices);
