@@ -139,6 +139,22 @@ def test_prefill_projection_shapes(torch_cuda, hidden, intermediate, vocabulary,
     _run_sequence(model, backend, 16, [prompt[:3], prompt[3:], prompt[:1]], table)
 
 
+@pytest.mark.parametrize("group", [1, 4])
+def test_prefill_scores_of_other_groups(torch_cuda, group):
+    """64-wide heads with 1 and 4 query heads per KV head: the row blocks'
+    scores are dealt to work-groups by (row, head), with blocks of fewer
+    row-heads than work-groups (2 rows of one head), full ones and a ragged
+    last one, across a 256-token chunk of the scores, bit for bit."""
+    cfg = tiny_config(hidden=64 * group, intermediate=64, heads=group, kv_heads=1, vocabulary=128, context=320, tied=1)
+    model = OracleModel(cfg, seed=37, stddev=0.08)
+    backend = HipBackend(cfg, block_tokens=16, max_blocks=20, max_sequences=1)
+    upload_model(backend, model)
+    o = Oracle()
+    prompt = [int(t) for t in o.fill_tokens(300, 37, 3400, 128)]
+    table = o.permutation(20, 37, 3401).copy()
+    _run_sequence(model, backend, 16, [prompt[:2], prompt[2:35], prompt[35:240], prompt[240:283], prompt[:1]], table)
+
+
 def test_batched_rows_match_single_sequences(torch_cuda):
     """Several sequences in one forward call == each appended alone."""
     cfg = smollm_config(layers=2, context=256)

@@ -26,6 +26,7 @@
 #include "exact_math.h"
 #include "kernels.h"
 #include "layout.h"
+#include "ordered_sum.h"
 
 namespace mphip {
 namespace {
@@ -182,6 +183,108 @@ __global__ __launch_bounds__(kScoreChunk) void attn_scores_kernel(const float* _
     }
 }
 
+// The scores of row blocks with 16-token pages and 64-wide heads: the work of
+// attn_scores_kernel with a block's row-heads dealt over grid z and q as
+// scalar operands. q of a (row, head) is the same for every lane, so it is
+// read with scalar loads, half a row ahead, and the arithmetic (one
+// v_mul_f32 with a scalar operand and one v_add_f32 per dim) is what bounds
+// the kernel; as LDS broadcasts q took more LDS cycles than the arithmetic
+// took, and one work-group per 48 row-heads left most SIMDs idle.
+// 256 rows at position 256 (96 (block, KV head, chunk) items): 36.6 -> 11.8 us;
+// 30 rows at 100: 33.8 -> 6.5.
+// The row-heads are dealt to 16 work-groups where that makes at most 1,536
+// (6 per CU), else to 8 or 4: 16, 8 and 4 took 11.8, 12.3 and 15.2 us with 96
+// items, 6.5, 8.0 and 11.5 with 6, but 68.6, 58.9 and 54.6 with 948 (each
+// work-group reads its K rows for itself).
+inline int score_parts(int items) {
+    int parts = 16;
+    while (parts > 4 && items * parts > 1536) parts /= 2;
+    return parts;
+}
+
+__global__ __launch_bounds__(kScoreChunk) void attn_scores_rows_kernel(const float* __restrict__ qkv, int ldq,
+                                                                       int heads, int kv_heads, RowMeta meta,
+                                                                       PagedKv kv, int layer, AttentionWork w) {
+    constexpr int DIM = 64, BT = 16, kHalf = DIM / 8;  // quads per half row
+    typedef const __attribute__((address_space(4))) f4v* ScalarQuad;
+    __shared__ float partial[kScoreChunk / 64][kMaxRowHeads];
+    const int2 item = w.items[blockIdx.x];
+    const int2 blk = w.blocks[item.x];
+    const int kvh = blockIdx.y, chunk = item.y;
+    const int r0 = blk.x, group = heads / kv_heads, rh = blk.y * group;
+    const int per = (rh + (int)gridDim.z - 1) / (int)gridDim.z;
+    const int i0 = blockIdx.z * per, i1 = min(rh, i0 + per);  // this work-group's row-heads
+    if (i0 >= i1) return;
+    const int pos0 = meta.row_pos[r0];
+    const int last_length = pos0 + blk.y;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int32_t* table = kv.tables + (size_t)meta.seq_slot[meta.row_seq[r0]] * kv.table_stride;
+    const int t = chunk * kScoreChunk + tid;
+    const bool live = t < last_length;
+    const int tc = live ? t : last_length - 1;
+    const float* kbase = kv.keys + kv_page_base(table[tc / BT], layer, kv.layers, BT, kv.kv_width) +
+                         key_offset(tc % BT, kvh, 0, BT, DIM);
+    f4v k[DIM / 4];
+#pragma unroll
+    for (int c = 0; c < DIM / 4; ++c) k[c] = *reinterpret_cast<const f4v*>(kbase + (size_t)c * BT * 4);
+    // Row-head i's q: quads 1 KB apart in the quad layout.
+    auto q_row = [&](int i) {
+        const int r = i / group, h = i - r * group;
+        return (uint64_t)(qkv + quad_index(r0 + r, (kvh * group + h) * DIM, ldq));
+    };
+    f4v qn[kHalf];
+    auto load = [&](uint64_t row, int half) {
+        // (The empty asm keeps the compiler from merging loads across runs.)
+        asm volatile("" : "+s"(row));
+#pragma unroll
+        for (int c = 0; c < kHalf; ++c) qn[c] = ((ScalarQuad)row)[(half * kHalf + c) * 64];
+    };
+    uint64_t row = q_row(i0);
+    load(row, 0);
+    const float root = sqrtf((float)DIM);
+    for (int i = i0; i < i1; ++i) {
+        const uint64_t next = q_row(min(i + 1, i1 - 1));
+        float acc = 0.0f;
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            f4v q[kHalf];
+#pragma unroll
+            for (int c = 0; c < kHalf; ++c) q[c] = qn[c];
+            // This half's q has arrived; only then the next half is
+            // requested (scalar loads return in any order).
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt 0
+            __builtin_amdgcn_sched_barrier(0);
+            if (half == 0) load(row, 1);
+            else load(next, 0);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int c = 0; c < kHalf; ++c) {
+                const f4v kc = k[half * kHalf + c];
+                acc = acc + q[c].x * kc.x;
+                acc = acc + q[c].y * kc.y;
+                acc = acc + q[c].z * kc.z;
+                acc = acc + q[c].w * kc.w;
+            }
+            asm volatile("" : "+v"(acc));  // the arithmetic stays before the next wait
+        }
+        row = next;
+        const int r = i / group, h = i - r * group;
+        const float score = acc / root;
+        const bool keep = live && t <= pos0 + r;
+        if (keep) w.scores[((size_t)(r0 + r) * heads + kvh * group + h) * w.stride + t] = score;
+        const float m = wave_max(keep ? score : -INFINITY);
+        if (lane == 0) partial[wave][i] = m;
+    }
+    __syncthreads();
+    if (tid < i1 - i0) {
+        const int i = i0 + tid, r = i / group, h = i - r * group;
+        float m = partial[0][i];
+#pragma unroll
+        for (int j = 1; j < kScoreChunk / 64; ++j) m = fmaxf(m, partial[j][i]);
+        w.chunk_max[((size_t)(r0 + r) * heads + kvh * group + h) * w.chunks + chunk] = m;
+    }
+}
+
 // One single-wavefront work-group per task: P heads (P = 1 for decode, the
 // whole group for prefill) of one row. It forms the row's softmax and its
 // output chains (lane = d):
@@ -269,9 +372,13 @@ __global__ __launch_bounds__(64) void attn_pv_kernel(int heads, int kv_heads, in
             }
         }
     };
-    // Lane h < P adds head h's staged e_t (tokens [0, n)) in order.
+    // Adds the staged e_t (tokens [0, n)) to the denominators in order: one
+    // head's with the whole wavefront (ordered_sum.h), several by lane h < P
+    // for head h.
     auto chain = [&](int n, float& den) {
-        if (lane < P) {
+        if constexpr (P == 1) {
+            den = ordered_sum(reinterpret_cast<const float*>(p_s[0]), n, den);
+        } else if (lane < P) {
             const float4* e4 = p_s[lane];
             const int full = n >> 2;
             int q = 0;
@@ -800,21 +907,30 @@ hipError_t launch_fused_decode(hipStream_t s, const float* qkv, int ldq, int hea
     return hipGetLastError();
 }
 
+constexpr int kPvApart = 1024;
+
 template <int BT, int DIM>
 hipError_t launch_pair(hipStream_t s, const float* qkv, int ldq, int heads, int kv_heads, int dim,
                        const RowMeta& meta, const PagedKv& kv, int layer, float* out, int ldo,
                        const AttentionWork& w, bool decode, const LaunchEvents& ev) {
-    launch_timed(attn_scores_kernel<BT, DIM>, dim3(w.items_count, kv_heads), dim3(kScoreChunk), s, ev.start, nullptr,
-                 qkv, ldq, heads, kv_heads, dim, meta, kv, layer, w, RopeTables{nullptr, nullptr});
     const int group = heads / kv_heads;
+    if constexpr (BT == 16 && DIM == 64)
+        launch_timed(attn_scores_rows_kernel, dim3(w.items_count, kv_heads, decode ? 1 : score_parts(w.items_count * kv_heads)),
+                     dim3(kScoreChunk), s, ev.start, nullptr, qkv, ldq, heads, kv_heads, meta, kv, layer, w);
+    else
+        launch_timed(attn_scores_kernel<BT, DIM>, dim3(w.items_count, kv_heads), dim3(kScoreChunk), s, ev.start,
+                     nullptr, qkv, ldq, heads, kv_heads, dim, meta, kv, layer, w, RopeTables{nullptr, nullptr});
     const int block_rows = attention_row_block(heads, kv_heads, dim);
     const dim3 wg(64);
     if (decode) {
         launch_timed(attn_pv_kernel<BT, DIM, 1>, dim3(w.blocks_count, kv_heads, group), wg, s, nullptr, ev.stop, heads,
                      kv_heads, dim, meta, kv, layer, w, out, ldo);
     } else {
+        // A wavefront per query head while a wavefront per (row, KV head)
+        // would leave SIMDs idle (a head's chain alone, and V read once per
+        // head), else one for the KV head's heads: PVFIG.
         const dim3 grid(w.blocks_count, kv_heads, block_rows);
-        switch (group) {
+        switch (w.blocks_count * kv_heads * block_rows <= kPvApart ? 1 : group) {
         case 2: launch_timed(attn_pv_kernel<BT, DIM, 2>, grid, wg, s, nullptr, ev.stop, heads, kv_heads, dim, meta, kv, layer, w, out, ldo); break;
         case 3: launch_timed(attn_pv_kernel<BT, DIM, 3>, grid, wg, s, nullptr, ev.stop, heads, kv_heads, dim, meta, kv, layer, w, out, ldo); break;
         case 4: launch_timed(attn_pv_kernel<BT, DIM, 4>, grid, wg, s, nullptr, ev.stop, heads, kv_heads, dim, meta, kv, layer, w, out, ldo); break;
