@@ -10,12 +10,12 @@
 //
 // A row block is up to 16 consecutive rows (positions) of one sequence;
 // decode rows are blocks of one. Two kernels per layer:
-//   scores: one work-group per (row block, kv head, 256-token chunk), thread
+//   scores: work-groups per (row block, kv head, 256-token chunk), thread
 //           = token: every (row, head) of the block that sees the token gets
 //           its score; per-chunk maxima go beside the scores.
-//   pv:     one single-wavefront work-group per (row, head) task: the
-//           softmax (maximum, e_t, the sequential denominator, p_t) and the
-//           output chains, lane = d.
+//   pv:     one single-wavefront work-group per (row, head) or (row, kv
+//           head) task: the softmax (maximum, e_t, the sequential
+//           denominator, p_t) and the output chains, lane = d.
 // Blocks arrive sorted by decreasing length so the longest chains start
 // first.
 #include <hip/hip_ext.h>
@@ -307,6 +307,7 @@ __global__ __launch_bounds__(64) void attn_pv_kernel(int heads, int kv_heads, in
     __shared__ int32_t table_s[kMaxTable];
     __shared__ float4 p_s[P][kPWindow / 4];
     __shared__ float den_s[P];
+    __shared__ uint64_t exp_tab[32];  // a table in memory costs a round trip per exponential
     const int dim = DIM ? DIM : dim_rt;
     const int bt = BT ? BT : kv.block_tokens;
     const int2 blk = w.blocks[blockIdx.x];
@@ -324,6 +325,7 @@ __global__ __launch_bounds__(64) void attn_pv_kernel(int heads, int kv_heads, in
     const int pages = (len + bt - 1) / bt;
     const float* srow = w.scores + ((size_t)row * heads + h0) * w.stride;
     const int nc = (len + kScoreChunk - 1) / kScoreChunk;
+    if (lane < 32) exp_tab[lane] = kExp2Table[lane];
     // Page table and chunk maxima: loads go out 8 per lane at a time
     // (unrolled, clamped), one memory latency per 8.
     for (int i0 = 0; i0 < pages; i0 += 64 * 8) {
@@ -364,9 +366,9 @@ __global__ __launch_bounds__(64) void attn_pv_kernel(int heads, int kv_heads, in
                     if (e < n4) {
                         const float m = mx[h];
                         const int u = 4 * e;  // padding past n is never read
-                        p_s[h][e] = make_float4(ref_expf(t[j].x - m), u + 1 < n ? ref_expf(t[j].y - m) : 0.0f,
-                                                u + 2 < n ? ref_expf(t[j].z - m) : 0.0f,
-                                                u + 3 < n ? ref_expf(t[j].w - m) : 0.0f);
+                        auto ex = [&](float s) { return ref_expf_select(s - m, exp_tab); };
+                        p_s[h][e] = make_float4(ex(t[j].x), u + 1 < n ? ex(t[j].y) : 0.0f,
+                                                u + 2 < n ? ex(t[j].z) : 0.0f, u + 3 < n ? ex(t[j].w) : 0.0f);
                     }
                 }
             }
@@ -907,7 +909,7 @@ hipError_t launch_fused_decode(hipStream_t s, const float* qkv, int ldq, int hea
     return hipGetLastError();
 }
 
-constexpr int kPvApart = 1024;
+constexpr int kPvApartTasks = 512, kPvApartLength = 1024;
 
 template <int BT, int DIM>
 hipError_t launch_pair(hipStream_t s, const float* qkv, int ldq, int heads, int kv_heads, int dim,
@@ -926,11 +928,14 @@ hipError_t launch_pair(hipStream_t s, const float* qkv, int ldq, int heads, int 
         launch_timed(attn_pv_kernel<BT, DIM, 1>, dim3(w.blocks_count, kv_heads, group), wg, s, nullptr, ev.stop, heads,
                      kv_heads, dim, meta, kv, layer, w, out, ldo);
     } else {
-        // A wavefront per query head while a wavefront per (row, KV head)
-        // would leave SIMDs idle (a head's chain alone, and V read once per
-        // head), else one for the KV head's heads: PVFIG.
+        // A wavefront per query head (its own e_t and chain, V read once per
+        // head) where few rows leave SIMDs idle or rows are long, else one for
+        // the KV head's heads. Apart against together: 7.5 vs 12.4 us for 30
+        // rows at position 100, 127 vs 134 for 256 rows at 3,000 and 128 vs
+        // 135 for 1,024 at 1,000, but 25.5 vs 24.2 for 256 at 256.
+        const bool apart = w.blocks_count * kv_heads * block_rows <= kPvApartTasks || w.stride > kPvApartLength;
         const dim3 grid(w.blocks_count, kv_heads, block_rows);
-        switch (w.blocks_count * kv_heads * block_rows <= kPvApart ? 1 : group) {
+        switch (apart ? 1 : group) {
         case 2: launch_timed(attn_pv_kernel<BT, DIM, 2>, grid, wg, s, nullptr, ev.stop, heads, kv_heads, dim, meta, kv, layer, w, out, ldo); break;
         case 3: launch_timed(attn_pv_kernel<BT, DIM, 3>, grid, wg, s, nullptr, ev.stop, heads, kv_heads, dim, meta, kv, layer, w, out, ldo); break;
         case 4: launch_timed(attn_pv_kernel<BT, DIM, 4>, grid, wg, s, nullptr, ev.stop, heads, kv_heads, dim, meta, kv, layer, w, out, ldo); break;
