@@ -112,3 +112,27 @@ def test_row_kernel_denominators(torch_cuda, scale, equal):
     that grow evenly."""
     for length in (500, 5000):
         _check(torch_cuda, Oracle(), 300, length, HEADS, KV_HEADS, scale, equal)
+
+
+@pytest.mark.parametrize("length", [1, 77, 503, 640, 1500, 5000])
+def test_out_in_place_of_q(torch_cuda, length):
+    """`out` may be q's own buffer: the work-groups of a head that read its q
+    must not find another's output there. Bits of the oracle, with more heads
+    (96, four work-groups each in the row kernel) than fit the chip at once,
+    so that some start after others have ended."""
+    torch, o = torch_cuda, Oracle()
+    heads, kv_heads = (96, 32) if length <= 2000 else (HEADS, KV_HEADS)
+    pages = math.ceil(length / BT)
+    kvw = kv_heads * DIM
+    keys, values = o.fill_normal(pages * BT * kvw, 400, 1), o.fill_normal(pages * BT * kvw, 400, 2)
+    q = o.fill_normal(heads * DIM, 400, 3)
+    table = o.permutation(pages, 400, 4)
+    want = o.attention(q, keys, values, table, length - 1, 1, 0, 1, BT, heads, kv_heads, DIM)[0]
+    dk, dv, dt = (torch.from_numpy(a).cuda() for a in (keys, values, table))
+    for call in (paged_attention_decode, paged_attention_decode_noalloc):
+        buffer = torch.from_numpy(q.copy()).cuda()
+        call(buffer.data_ptr(), dk.data_ptr(), dv.data_ptr(), dt.data_ptr(), length, 0, 1, BT, heads, kv_heads, DIM,
+             buffer.data_ptr(), None)
+        torch.cuda.synchronize()
+        got = buffer.cpu().numpy()
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (call.__name__, length)

@@ -578,7 +578,15 @@ hipError_t launch_attention_single(hipStream_t s, const float* q, const float* k
                                    int layer, int layers, int block_tokens, int heads,
                                    int kv_heads, int dim, float* out, float* scratch) {
     if (heads / kv_heads > kMaxGroup || dim > kMaxDim || dim % 4) return hipErrorInvalidValue;
-    if (block_tokens == kRowPage && dim == kRowDim && (scratch || length <= kRowWindow)) {
+    // The row kernel's work-groups of one head read the whole head's q and each
+    // writes its own dims of out, so where the scores are formed there and out
+    // lies over q, one would read what another has written. attention_single's
+    // work-group reads its heads' q before it writes them, and no other
+    // work-group touches them: such calls take it.
+    const size_t width = (size_t)heads * dim;
+    const bool over_q = (uintptr_t)out < (uintptr_t)(q + width) && (uintptr_t)q < (uintptr_t)(out + width);
+    const bool scores_first = scratch && length > kScoresInRow;
+    if (block_tokens == kRowPage && dim == kRowDim && (scratch || length <= kRowWindow) && (scores_first || !over_q)) {
         const RowArgs a{q, keys, values, table, length, layer, layers, heads, kv_heads, out, scratch};
         switch (heads / kv_heads) {
         case 1: launch_row<1>(s, a); break;
