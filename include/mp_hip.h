@@ -189,12 +189,13 @@ int mp_hip_paged_attention_decode_fast(const float* q, const float* keys, const 
 /* The same attention as mp_hip_paged_attention_decode with no allocation of
  * any kind: no counterpart in the reference; for callers that cannot
  * allocate (code under HIP graph capture, serving loops that forbid
- * allocation). The scores of a long row go to a 1 MiB device array of the
- * library (one per GPU, held until the process ends) instead of a per-call
+ * allocation). The scores of a long row (heads / kv_heads *
+ * round_up(length, 16) > 10240) go to a 1 MiB device array of the library
+ * (one per GPU, held until the process ends) instead of a per-call
  * hipMalloc; a row must satisfy heads * round_up(length, 16) <= 262144, or
  * the call returns MP_INVALID_ARGUMENT (message: mp_hip_last_error(NULL)).
- * Calls that overlap on one GPU share the array and race. Asynchronous on
- * `stream`. */
+ * Calls for long rows that overlap on one GPU share the array and race;
+ * others may overlap. Asynchronous on `stream`. */
 int mp_hip_paged_attention_decode_noalloc(const float* q, const float* keys, const float* values,
                                           const int32_t* table, int32_t length, int32_t layer,
                                           int32_t layers, int32_t block_tokens, int32_t heads,

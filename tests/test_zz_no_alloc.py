@@ -6,7 +6,7 @@ Two calls in a row on rows long enough that their scores leave LDS for the
 static device scratch (a KV head's 3 query heads x round_up(length, 16) >
 kAttentionLdsScores = 10,240 floats), the second shorter than the first, so
 it runs over what the first left there; then a row of 100 tokens, whose
-scores stay in LDS although the entry point passes the scratch as well.
+scores stay in LDS.
 Outputs must be bit-identical to the allocating entry point's (and to the
 oracle's: the kernel keeps the reference CPU path's order). A row beyond
 the scratch is rejected before any launch."""
@@ -91,8 +91,9 @@ def _check(torch, o, seed, length, heads, kv_heads, scale=1.0, equal_keys=False)
 def test_row_kernel_edges(torch_cuda, length):
     """Bits of the oracle at the edges of the row kernel: partial pages,
     phases of 14 pages and turns of four phases, the 256 denominator values
-    added one by one, rows whose scores take a launch of their own (over 640
-    tokens, in the scratch), and rows beyond the 18,432-token window."""
+    added one by one, rows whose scores take a launch of their own (from 3,409
+    tokens on with 3 query heads per KV head, in the scratch), and rows beyond
+    the 18,432-token window."""
     _check(torch_cuda, Oracle(), 100 + length, length, HEADS, KV_HEADS)
 
 
@@ -100,7 +101,7 @@ def test_row_kernel_edges(torch_cuda, length):
 def test_row_kernel_groups(torch_cuda, group):
     """Every number of query heads per KV head, scores in the row kernel and
     in the scratch."""
-    for length in (77, 1500):
+    for length in (77, 1500, 10300):
         _check(torch_cuda, Oracle(), 200 + group, length, 2 * group, 2)
 
 
@@ -136,3 +137,26 @@ def test_out_in_place_of_q(torch_cuda, length):
         torch.cuda.synchronize()
         got = buffer.cpu().numpy()
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (call.__name__, length)
+
+
+def test_rows_with_scores_on_the_chip_may_overlap(torch_cuda):
+    """Allocation-free calls for rows of up to 10,240 score floats per KV head
+    share nothing: eight rows of 700 to 3,408 tokens on eight streams at once,
+    ten rounds, each with the oracle's bits."""
+    torch, o = torch_cuda, Oracle()
+    rows = []
+    for i, length in enumerate((700, 1000, 1500, 2000, 2500, 3000, 3400, 3408)):
+        q, keys, values, table = _inputs(o, 500 + i, length)
+        want = o.attention(q, keys, values, table, length - 1, 1, LAYER, LAYERS, BT, HEADS, KV_HEADS, DIM)[0]
+        rows.append((length, [torch.from_numpy(a).cuda() for a in (q, keys, values, table)], want,
+                     torch.empty(HEADS * DIM, dtype=torch.float32, device="cuda"), torch.cuda.Stream()))
+    for _ in range(10):
+        for _, _, _, out, _ in rows:
+            out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        for length, inputs, _, out, stream in rows:
+            paged_attention_decode_noalloc(*(t.data_ptr() for t in inputs), length, LAYER, LAYERS, BT, HEADS, KV_HEADS,
+                                           DIM, out.data_ptr(), stream.cuda_stream)
+        torch.cuda.synchronize()
+        for length, _, want, out, _ in rows:
+            assert np.array_equal(out.cpu().numpy().view(np.uint32), want.view(np.uint32)), length

@@ -7,9 +7,13 @@
 // memory it allocates per call. Here that buffer is `scratch`, a
 // file-scope device array of kScratchFloats floats (1 MiB) that every GPU
 // running the library holds until the process ends. A row fits when
-// heads * round_up(length, 16) <= kScratchFloats. The kernel writes every
-// score slot before reading it, so the array needs no clearing between
-// calls; calls that overlap on one GPU share it and race.
+// heads * round_up(length, 16) <= kScratchFloats. Only rows whose scores the
+// allocating call would keep in global memory use the array
+// (attention_scores_global): calls that overlap on one GPU share it and race,
+// and shorter rows may overlap. (The array for every row over 640 tokens gave
+// 20.1 instead of 25.4 us for one of 1,000, but two of them on two streams
+// could overwrite each other's scores.) The kernels write every score slot
+// before reading it, so the array needs no clearing between calls.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -81,11 +85,13 @@ extern "C" int mp_hip_paged_attention_decode_noalloc(const float* q, const float
         return MP_INVALID_ARGUMENT;
     }
     float* buffer = nullptr;
-    std::string error;
-    const int status = scratch_for_current_device(&buffer, &error);
-    if (status) {
-        mphip::set_free_error(error);
-        return status;
+    if (mphip::attention_scores_global(heads / kv_heads, length)) {
+        std::string error;
+        const int status = scratch_for_current_device(&buffer, &error);
+        if (status) {
+            mphip::set_free_error(error);
+            return status;
+        }
     }
     const hipError_t e = mphip::launch_attention_single(static_cast<hipStream_t>(stream), q, keys, values, table,
                                                         length, layer, layers, block_tokens, heads, kv_heads, dim,

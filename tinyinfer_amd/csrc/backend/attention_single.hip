@@ -259,7 +259,7 @@ __global__ __launch_bounds__(kAttentionThreads) void attention_single_kernel(
 // bytes one CU can read (about 15 of the 64 per clock it nominally takes,
 // over scattered rows). So:
 // - scores (parallel over tokens): in a kernel of their own over the whole
-//   chip when a row is long and scratch is there, else in the row kernel;
+//   chip where the row has scratch, else in the row kernel;
 // - the row kernel: one work-group per query head and 16 of its dims, so that
 //   a CU streams a quarter of the head's V. Each forms e_t and p_t for itself
 //   with all wavefronts and the denominator by ordered_sum (a fifth of its
@@ -556,18 +556,12 @@ __global__ __launch_bounds__(kRowThreads) void attention_row_kernel(RowArgs a) {
     if (wave == 0 && lane < kSlice) a.out[(size_t)head * kRowDim + d0 + lane] = total;
 }
 
-// Rows of more than this many tokens compute their scores over the whole chip
-// first (when there is scratch for them), for one more launch: in the row
-// kernel they take 3.1 us at 64 tokens, 7.2 at 503 and 12.2 at 1,024, read
-// from the scratch 1.6 us after a launch of 6 to 7.5.
-constexpr int kScoresInRow = 640;
-
 template <int G>
-void launch_row(hipStream_t s, RowArgs a) {
-    if (a.scores && a.length > kScoresInRow)
+void launch_row(hipStream_t s, const RowArgs& a) {
+    // In the row kernel the scores take 3.1 us at 64 tokens, 7.2 at 503 and
+    // 12.2 at 1,024; read from the scratch 1.6 us after a launch of 6 to 7.5.
+    if (a.scores)
         attention_row_scores_kernel<G><<<dim3((a.length + kScoreThreads - 1) / kScoreThreads, a.kv_heads), kScoreThreads, 0, s>>>(a);
-    else
-        a.scores = nullptr;
     attention_row_kernel<<<a.heads * (kRowDim / kSlice), kRowThreads, 0, s>>>(a);
 }
 
@@ -585,8 +579,7 @@ hipError_t launch_attention_single(hipStream_t s, const float* q, const float* k
     // work-group touches them: such calls take it.
     const size_t width = (size_t)heads * dim;
     const bool over_q = (uintptr_t)out < (uintptr_t)(q + width) && (uintptr_t)q < (uintptr_t)(out + width);
-    const bool scores_first = scratch && length > kScoresInRow;
-    if (block_tokens == kRowPage && dim == kRowDim && (scratch || length <= kRowWindow) && (scores_first || !over_q)) {
+    if (block_tokens == kRowPage && dim == kRowDim && (scratch || (length <= kRowWindow && !over_q))) {
         const RowArgs a{q, keys, values, table, length, layer, layers, heads, kv_heads, out, scratch};
         switch (heads / kv_heads) {
         case 1: launch_row<1>(s, a); break;

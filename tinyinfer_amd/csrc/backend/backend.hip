@@ -1458,7 +1458,7 @@ int mp_hip_paged_attention_decode(const float* q, const float* keys, const float
     const int group = heads / kv_heads;
     float* scratch = nullptr;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if ((size_t)group * (size_t)((length + 15) & ~15) > (size_t)mphip::kAttentionLdsScores) {
+    if (mphip::attention_scores_global(group, length)) {
         // Long rows keep their scores in global memory; synchronous so the
         // temporary can be released before returning.
         const size_t floats = (size_t)kv_heads * group * (size_t)((length + 15) & ~15);

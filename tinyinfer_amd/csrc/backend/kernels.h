@@ -7,6 +7,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "launch_rules.h"
+
 namespace mphip {
 
 // Per-call row metadata resident on the device. Row r of a forward call is
@@ -342,11 +344,11 @@ hipError_t launch_attention(hipStream_t s, float* qkv, int ldq, int rows, int he
                             const AttentionWork& work, bool decode, const RopeTables& rope,
                             const LaunchEvents& events = LaunchEvents());
 // Stand-alone single-row variant over a caller page table (plain layouts).
+// `scratch`: heads * round_up(length, 16) floats where
+// attention_scores_global(heads / kv_heads, length), else null.
 hipError_t launch_attention_single(hipStream_t s, const float* q, const float* keys, const float* values,
                                    const int32_t* table, int length, int layer, int layers, int block_tokens,
                                    int heads, int kv_heads, int dim, float* out, float* scratch);
-// Score floats per row that fit in LDS.
-constexpr int kAttentionLdsScores = 10240;
 
 // One copy-on-write: the first `valid` token slots of page `source` into
 // page `destination` (block ids), every layer, both pools.
