@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "../../../include/mp_hip.h"
+#include "idle_memory.h"
 #include "kernels.h"
 #include "layout.h"
 
@@ -466,19 +467,34 @@ struct FreeWork {
 std::mutex g_free_work_mutex;
 FreeWork g_free_work[kFreeWorkSets];  // the sets with a device pointer are idle
 
+struct DeviceMemory {
+    static int allocate(void** out, size_t bytes) { return hipMalloc(out, bytes); }
+    static void clear_error() { (void)hipGetLastError(); }
+};
+struct PinnedMemory {
+    static int allocate(void** out, size_t bytes) { return hipHostMalloc(out, bytes, hipHostMallocDefault); }
+    static void clear_error() { (void)hipGetLastError(); }
+};
+
 void release_free_work(FreeWork& work) {
     if (work.device) (void)hipFree(work.device);
     if (work.host) (void)hipHostFree(work.host);
     work = FreeWork{};
 }
 
-void trim_free_work() {
+// Frees the idle sets; whether there was one.
+bool trim_free_work() {
     FreeWork idle[kFreeWorkSets];
     {
         std::lock_guard<std::mutex> lock(g_free_work_mutex);
         std::swap(idle, g_free_work);
     }
-    for (FreeWork& work : idle) release_free_work(work);
+    bool any = false;
+    for (FreeWork& work : idle) {
+        any |= work.device != nullptr;
+        release_free_work(work);
+    }
+    return any;
 }
 
 hipError_t take_free_work(size_t device_bytes, size_t host_bytes, FreeWork* out) {
@@ -499,16 +515,11 @@ hipError_t take_free_work(size_t device_bytes, size_t host_bytes, FreeWork* out)
     work.gpu = gpu;
     work.device_bytes = round(device_bytes);
     work.host_bytes = round(host_bytes);
-    for (int attempt = 0; attempt < 2; ++attempt) {
-        e = work.device ? hipSuccess : hipMalloc(&work.device, work.device_bytes);
-        if (e == hipSuccess) e = hipHostMalloc(&work.host, work.host_bytes, hipHostMallocDefault);
-        if (e == hipSuccess) {
-            *out = work;
-            return e;
-        }
-        if (attempt == 0) trim_free_work();
-    }
-    release_free_work(work);
+    e = (hipError_t)mphip::allocate_with_room<DeviceMemory>((void**)&work.device, work.device_bytes, trim_free_work);
+    if (e == hipSuccess)
+        e = (hipError_t)mphip::allocate_with_room<PinnedMemory>((void**)&work.host, work.host_bytes, trim_free_work);
+    if (e == hipSuccess) *out = work;
+    else release_free_work(work);
     return e;
 }
 
@@ -1537,7 +1548,6 @@ int mp_hip_paged_attention_decode_fast(const float* q, const float* keys, const 
     FreeWork work;
     hipError_t e = take_free_work(int_bytes + partial_floats * sizeof(float), int_bytes, &work);
     if (e != hipSuccess) {
-        (void)hipGetLastError();
         mphip::set_free_error(std::string("allocate fast attention work: ") + hipGetErrorString(e));
         return e == hipErrorOutOfMemory ? MP_OUT_OF_MEMORY : MP_DEVICE_ERROR;
     }
