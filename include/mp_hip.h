@@ -179,8 +179,10 @@ int mp_hip_paged_attention_decode(const float* q, const float* keys, const float
  * major, K as [d/4][slot][4], V as [slot/4][d][4]), not the reference's
  * [slot][kv_width]. Needs block_tokens 16, dim 64 and at most 4 query heads
  * per KV head, else MP_INVALID_ARGUMENT (message:
- * mp_hip_last_error(NULL)). Allocates its work lists and partials per call
- * and is synchronous on `stream` (NULL: the null stream). */
+ * mp_hip_last_error(NULL)). Its work lists and partials come from memory that
+ * the library keeps between calls (at most 256 MiB of device and as much of
+ * pinned memory; destroying any context frees it). Synchronous on `stream`
+ * (NULL: the null stream). */
 int mp_hip_paged_attention_decode_fast(const float* q, const float* keys, const float* values,
                                        const int32_t* tables, int32_t table_stride, const int32_t* lengths,
                                        int32_t rows, int32_t layer, int32_t layers, int32_t block_tokens,

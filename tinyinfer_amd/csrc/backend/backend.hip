@@ -14,11 +14,9 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
-#include <mutex>
 #include <new>
 #include <string>
 #include <unordered_map>
-#include <utility>
 #include <vector>
 
 #include "../../../include/mp_hip.h"
@@ -451,88 +449,38 @@ void set_free_error(const std::string& message) { g_free_error = message; }
 
 namespace {
 
-// Device and pinned memory of the context-free fast attention: a call takes a
-// set for itself (any thread, any stream) and puts it back after it has
-// waited for its stream, so an idle set is in nobody's use. At most
-// kFreeWorkSets stay, of at most kFreeWorkBytes each; destroying a context,
-// and a call that finds no memory, gives them back. (A call of 64 rows of
-// 300 to 2,000 tokens: 95 -> 56 us without an allocation of its own.)
-constexpr size_t kFreeWorkSets = 4, kFreeWorkBytes = 64u << 20;
-struct FreeWork {
-    char* device = nullptr;
-    int32_t* host = nullptr;  // pinned
-    size_t device_bytes = 0, host_bytes = 0;
-    int gpu = -1;
-};
-std::mutex g_free_work_mutex;
-FreeWork g_free_work[kFreeWorkSets];  // the sets with a device pointer are idle
-
 struct DeviceMemory {
     static int allocate(void** out, size_t bytes) { return hipMalloc(out, bytes); }
+    static void release(void* p) { (void)hipFree(p); }
     static void clear_error() { (void)hipGetLastError(); }
 };
 struct PinnedMemory {
     static int allocate(void** out, size_t bytes) { return hipHostMalloc(out, bytes, hipHostMallocDefault); }
+    static void release(void* p) { (void)hipHostFree(p); }
     static void clear_error() { (void)hipGetLastError(); }
 };
 
-void release_free_work(FreeWork& work) {
-    if (work.device) (void)hipFree(work.device);
-    if (work.host) (void)hipHostFree(work.host);
-    work = FreeWork{};
+// Work memory of the context-free fast attention between its calls (64 rows
+// of 300 to 2,000 tokens: 95 -> 56 us without an allocation in the call). A
+// call puts its memory back after it has waited for its stream. Destroying a
+// context, and a call that finds no memory, frees what is idle. The pinned
+// lists and the device memory (lists and partials) are kept apart: a call
+// whose partials are too large to keep allocates no pinned memory either.
+mphip::IdleMemory<DeviceMemory> g_idle_device;
+mphip::IdleMemory<PinnedMemory> g_idle_pinned;
+
+bool trim_idle_memory() {
+    const bool device = g_idle_device.trim(), pinned = g_idle_pinned.trim();
+    return device || pinned;
 }
 
-// Frees the idle sets; whether there was one.
-bool trim_free_work() {
-    FreeWork idle[kFreeWorkSets];
-    {
-        std::lock_guard<std::mutex> lock(g_free_work_mutex);
-        std::swap(idle, g_free_work);
-    }
-    bool any = false;
-    for (FreeWork& work : idle) {
-        any |= work.device != nullptr;
-        release_free_work(work);
-    }
-    return any;
-}
-
-hipError_t take_free_work(size_t device_bytes, size_t host_bytes, FreeWork* out) {
-    int gpu = 0;
-    hipError_t e = hipGetDevice(&gpu);
-    if (e != hipSuccess) return e;
-    {
-        std::lock_guard<std::mutex> lock(g_free_work_mutex);
-        for (FreeWork& work : g_free_work)
-            if (work.device && work.gpu == gpu && work.device_bytes >= device_bytes && work.host_bytes >= host_bytes) {
-                *out = work;
-                work = FreeWork{};
-                return hipSuccess;
-            }
-    }
-    auto round = [](size_t bytes) { return (bytes + (1u << 20) - 1) >> 20 << 20; };
-    FreeWork work;
-    work.gpu = gpu;
-    work.device_bytes = round(device_bytes);
-    work.host_bytes = round(host_bytes);
-    e = (hipError_t)mphip::allocate_with_room<DeviceMemory>((void**)&work.device, work.device_bytes, trim_free_work);
-    if (e == hipSuccess)
-        e = (hipError_t)mphip::allocate_with_room<PinnedMemory>((void**)&work.host, work.host_bytes, trim_free_work);
-    if (e == hipSuccess) *out = work;
-    else release_free_work(work);
-    return e;
-}
-
-void put_free_work(FreeWork& work, bool idle) {
-    if (idle && work.device_bytes <= kFreeWorkBytes && work.host_bytes <= kFreeWorkBytes) {
-        std::lock_guard<std::mutex> lock(g_free_work_mutex);
-        for (FreeWork& slot : g_free_work)
-            if (!slot.device) {
-                slot = work;
-                return;
-            }
-    }
-    release_free_work(work);
+template <typename Memory>
+hipError_t take_idle_memory(mphip::IdleMemory<Memory>& idle, int gpu, size_t bytes,
+                            typename mphip::IdleMemory<Memory>::Buffer* out) {
+    if (idle.take(gpu, bytes, out)) return hipSuccess;
+    out->bytes = (bytes + (1u << 20) - 1) >> 20 << 20;
+    out->gpu = gpu;
+    return (hipError_t)mphip::allocate_with_room<Memory>(&out->data, out->bytes, trim_idle_memory);
 }
 
 }  // namespace
@@ -656,7 +604,7 @@ int mp_hip_destroy(mp_hip* h) {
         if (p) (void)hipFree(p);
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
-    trim_free_work();
+    (void)trim_idle_memory();
     return MP_OK;
 }
 
@@ -1545,21 +1493,26 @@ int mp_hip_paged_attention_decode_fast(const float* q, const float* keys, const 
     const size_t int_bytes = (ints * sizeof(int32_t) + 255) / 256 * 256;
     const size_t partial_floats = (size_t)rows * kv_heads * max_splits * group * (64 + 2);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    FreeWork work;
-    hipError_t e = take_free_work(int_bytes + partial_floats * sizeof(float), int_bytes, &work);
+    int gpu = 0;
+    mphip::IdleMemory<DeviceMemory>::Buffer device;
+    mphip::IdleMemory<PinnedMemory>::Buffer pinned;
+    hipError_t e = hipGetDevice(&gpu);
+    if (e == hipSuccess) e = take_idle_memory(g_idle_device, gpu, int_bytes + partial_floats * sizeof(float), &device);
+    if (e == hipSuccess) e = take_idle_memory(g_idle_pinned, gpu, int_bytes, &pinned);
     if (e != hipSuccess) {
+        g_idle_device.put(device);
         mphip::set_free_error(std::string("allocate fast attention work: ") + hipGetErrorString(e));
         return e == hipErrorOutOfMemory ? MP_OUT_OF_MEMORY : MP_DEVICE_ERROR;
     }
-    int32_t* host = work.host;
+    int32_t* host = static_cast<int32_t*>(pinned.data);
     for (const std::vector<int32_t>* part : {&counts, (const std::vector<int32_t>*)&split_items,
                                              (const std::vector<int32_t>*)&short_items,
                                              (const std::vector<int32_t>*)&merge_rows,
                                              (const std::vector<int32_t>*)&positions})
         host = std::copy(part->begin(), part->end(), host);
-    char* const buffer = work.device;
+    char* const buffer = static_cast<char*>(device.data);
     int32_t* const dev = reinterpret_cast<int32_t*>(buffer);
-    e = hipMemcpyAsync(dev, work.host, ints * sizeof(int32_t), hipMemcpyHostToDevice, s);
+    e = hipMemcpyAsync(dev, pinned.data, ints * sizeof(int32_t), hipMemcpyHostToDevice, s);
     mphip::FastAttentionWork w{};
     w.items = dev + counts.size();
     w.items_count = w.items_capacity = counts[0];
@@ -1584,7 +1537,13 @@ int mp_hip_paged_attention_decode_fast(const float* q, const float* keys, const 
     // Synchronous, so that the work lists are idle when they are put back.
     const hipError_t done = hipStreamSynchronize(s);
     if (e == hipSuccess) e = done;
-    put_free_work(work, e == hipSuccess);
+    if (e == hipSuccess) {
+        g_idle_device.put(device);
+        g_idle_pinned.put(pinned);
+    } else {
+        DeviceMemory::release(device.data);
+        PinnedMemory::release(pinned.data);
+    }
     if (e != hipSuccess) {
         mphip::set_free_error(std::string("fast paged attention: ") + hipGetErrorString(e));
         return MP_DEVICE_ERROR;
