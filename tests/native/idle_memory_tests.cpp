@@ -149,6 +149,19 @@ void bounded() {
     CHECK(Runtime::live == 0);
 }
 
+// What is kept gives way to another allocation that finds no memory.
+void gives_way() {
+    Runtime::reset(0);
+    Pool pool;
+    CHECK(allocations_of(pool, 50 * kMiB) == 1 && Runtime::live == 1);
+    Runtime::failures = 1;
+    void* p = nullptr;
+    CHECK(allocate_with_room<Runtime>(&p, 16, [&] { return pool.trim(); }) == 0 && p && Runtime::live == 1);
+    Runtime::release(p);
+    Runtime::failures = 1;  // nothing left to give back
+    CHECK(allocate_with_room<Runtime>(&p, 16, [&] { return pool.trim(); }) == kOutOfMemory && Runtime::last_error == 0);
+}
+
 struct Quiet {
     static void release(void* p) { std::free(p); }
 };
@@ -187,6 +200,7 @@ int main() {
     growing_calls_allocate_once();
     smallest_that_fits();
     bounded();
+    gives_way();
     threads();
     std::puts("ok");
     return 0;

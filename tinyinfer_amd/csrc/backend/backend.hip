@@ -164,13 +164,44 @@ int stream_wait_polling(mp_hip* h, const char* what) {
     return check(h, e, what);
 }
 
+struct DeviceMemory {
+    static int allocate(void** out, size_t bytes) { return hipMalloc(out, bytes); }
+    static void release(void* p) { (void)hipFree(p); }
+    static void clear_error() { (void)hipGetLastError(); }
+};
+struct PinnedMemory {
+    static int allocate(void** out, size_t bytes) { return hipHostMalloc(out, bytes, hipHostMallocDefault); }
+    static void release(void* p) { (void)hipHostFree(p); }
+    static void clear_error() { (void)hipGetLastError(); }
+};
+
+// Work memory of the context-free fast attention between its calls (64 rows
+// of 300 to 2,000 tokens: 95 -> 56 us without an allocation in the call). A
+// call puts its memory back after it has waited for its stream. Destroying a
+// context, and any allocation that finds no memory, frees what is idle. The pinned
+// lists and the device memory (lists and partials) are kept apart: a call
+// whose partials are too large to keep allocates no pinned memory either.
+mphip::IdleMemory<DeviceMemory> g_idle_device;
+mphip::IdleMemory<PinnedMemory> g_idle_pinned;
+
+bool trim_idle_memory() {
+    const bool device = g_idle_device.trim(), pinned = g_idle_pinned.trim();
+    return device || pinned;
+}
+
+template <typename Memory>
+hipError_t take_idle_memory(mphip::IdleMemory<Memory>& idle, int gpu, size_t bytes,
+                            typename mphip::IdleMemory<Memory>::Buffer* out) {
+    if (idle.take(gpu, bytes, out)) return hipSuccess;
+    out->bytes = (bytes + (1u << 20) - 1) >> 20 << 20;
+    out->gpu = gpu;
+    return (hipError_t)mphip::allocate_with_room<Memory>(&out->data, out->bytes, trim_idle_memory);
+}
+
 int device_alloc(mp_hip* h, void** out, size_t bytes, const char* what) {
     void* p = nullptr;
-    const hipError_t e = hipMalloc(&p, bytes ? bytes : 4);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        return check(h, e, what);
-    }
+    const int e = mphip::allocate_with_room<DeviceMemory>(&p, bytes ? bytes : 4, trim_idle_memory);
+    if (e) return check(h, (hipError_t)e, what);
     h->allocations.push_back(p);
     ++h->stats.device_allocations;
     *out = p;
@@ -361,8 +392,8 @@ int ensure_pinned(mp_hip* h, int32_t** buffer, size_t* capacity, size_t entries,
     *buffer = nullptr;
     *capacity = 0;
     const size_t cap = entries + entries / 2;
-    if ((status = check(h, hipHostMalloc((void**)buffer, sizeof(int32_t) * cap, hipHostMallocDefault), what)))
-        return status;
+    const int e = mphip::allocate_with_room<PinnedMemory>((void**)buffer, sizeof(int32_t) * cap, trim_idle_memory);
+    if ((status = check(h, (hipError_t)e, what))) return status;
     *capacity = cap;
     return MP_OK;
 }
@@ -446,44 +477,6 @@ thread_local std::string g_free_error = "no error";
 }  // namespace
 void set_free_error(const std::string& message) { g_free_error = message; }
 }  // namespace mphip
-
-namespace {
-
-struct DeviceMemory {
-    static int allocate(void** out, size_t bytes) { return hipMalloc(out, bytes); }
-    static void release(void* p) { (void)hipFree(p); }
-    static void clear_error() { (void)hipGetLastError(); }
-};
-struct PinnedMemory {
-    static int allocate(void** out, size_t bytes) { return hipHostMalloc(out, bytes, hipHostMallocDefault); }
-    static void release(void* p) { (void)hipHostFree(p); }
-    static void clear_error() { (void)hipGetLastError(); }
-};
-
-// Work memory of the context-free fast attention between its calls (64 rows
-// of 300 to 2,000 tokens: 95 -> 56 us without an allocation in the call). A
-// call puts its memory back after it has waited for its stream. Destroying a
-// context, and a call that finds no memory, frees what is idle. The pinned
-// lists and the device memory (lists and partials) are kept apart: a call
-// whose partials are too large to keep allocates no pinned memory either.
-mphip::IdleMemory<DeviceMemory> g_idle_device;
-mphip::IdleMemory<PinnedMemory> g_idle_pinned;
-
-bool trim_idle_memory() {
-    const bool device = g_idle_device.trim(), pinned = g_idle_pinned.trim();
-    return device || pinned;
-}
-
-template <typename Memory>
-hipError_t take_idle_memory(mphip::IdleMemory<Memory>& idle, int gpu, size_t bytes,
-                            typename mphip::IdleMemory<Memory>::Buffer* out) {
-    if (idle.take(gpu, bytes, out)) return hipSuccess;
-    out->bytes = (bytes + (1u << 20) - 1) >> 20 << 20;
-    out->gpu = gpu;
-    return (hipError_t)mphip::allocate_with_room<Memory>(&out->data, out->bytes, trim_idle_memory);
-}
-
-}  // namespace
 
 extern "C" {
 
@@ -1421,7 +1414,8 @@ int mp_hip_paged_attention_decode(const float* q, const float* keys, const float
         // Long rows keep their scores in global memory; synchronous so the
         // temporary can be released before returning.
         const size_t floats = (size_t)kv_heads * group * (size_t)((length + 15) & ~15);
-        if (hipMalloc(&scratch, floats * sizeof(float)) != hipSuccess) return MP_OUT_OF_MEMORY;
+        if (mphip::allocate_with_room<DeviceMemory>((void**)&scratch, floats * sizeof(float), trim_idle_memory))
+            return MP_OUT_OF_MEMORY;
     }
     hipError_t e = mphip::launch_attention_single(s, q, keys, values, table, length, layer, layers,
                                                   block_tokens, heads, kv_heads, dim, out, scratch);
