@@ -4,6 +4,7 @@
 
 #include <cstdio>
 #include <cstdlib>
+#include <initializer_list>
 
 #define CHECK(condition)                                                                \
     do {                                                                                \
@@ -28,8 +29,27 @@ static void scores_in_global_memory() {
     CHECK(attention_scores_global(8, 2147483632));
 }
 
+// 64-row tiles where they fill the chip, and never for up to 32 rows, however
+// many columns there are.
+static void large_tiles() {
+    for (int rows : {1, 8, 16, 17, 32})
+        for (int columns = 64; columns <= 1 << 20; columns += 4032)
+            for (int cb : {1, 2}) CHECK(!fast_large_tiles(rows, columns, 4, cb));
+    CHECK(fast_large_tiles(33, 7168, 4, 1));   // 448 tiles
+    CHECK(!fast_large_tiles(33, 7152, 4, 1));  // 447
+    CHECK(!fast_large_tiles(64, 8192, 4, 2));  // 256 tiles of 32 columns
+    CHECK(fast_large_tiles(64, 14336, 4, 2));  // 448
+    CHECK(!fast_large_tiles(4096, 1552, 4, 2));  // 97 column blocks: no pairs
+    CHECK(fast_large_tiles(4096, 1552, 4, 1));
+    CHECK(!fast_large_tiles(512, 1536, 4, 2));  // the sizes measured beside the rule
+    CHECK(fast_large_tiles(512, 1536, 4, 1));
+    CHECK(!fast_large_tiles(512, 576, 4, 1));
+    CHECK(fast_large_tiles(2147483647 - 15, 1 << 20, 4, 2));
+}
+
 int main() {
     scores_in_global_memory();
+    large_tiles();
     std::puts("ok");
     return 0;
 }

@@ -379,6 +379,38 @@ def test_fast_head_rows_do_not_depend_on_the_passes(torch_cuda, count, vocabular
     assert np.array_equal(together.view(np.uint32), apart.view(np.uint32))
 
 
+@pytest.mark.parametrize("intermediate", [7168, 14336])
+def test_fast_wide_projection_rows_same_in_any_tile(torch_cuda, intermediate):
+    """Wide projections take 16-row tiles up to 32 rows and 64-row tiles of one
+    (7,168 columns) or two (14,336) column blocks from 33 rows on: 33 rows
+    decoded together, 32 and 7 of them, give the same logits, bit for bit,
+    within 1e-3 relative of the oracle."""
+    cfg = dict(layers=1, hidden=128, intermediate=intermediate, heads=2, kv_heads=1, vocabulary=256, context=32, eos=0,
+               rms_epsilon=1e-5, rope_theta=100000.0, tied=0)
+    model = OracleModel(cfg, seed=79, stddev=0.05)
+    o = Oracle()
+    rows = 33
+    tokens = [int(t) for t in o.fill_tokens(2 * rows, 79, 9900, 256)]
+    backend = HipBackend(cfg, block_tokens=16, max_blocks=rows, max_sequences=rows, arithmetic=ARITHMETIC_FAST)
+    upload_model(backend, model)
+    for i in range(rows):
+        backend.table_write(i, 0, np.array([i], dtype=np.int32))
+    backend.forward([(i, 0, 1) for i in range(rows)], tokens[:rows])
+    got = {}
+    for count in (rows, 32, 7):
+        _, logits = backend.forward([(i, 1, 1) for i in range(count)], tokens[rows:rows + count])
+        got[count] = logits.copy()
+    backend.close()
+    for count in (32, 7):
+        assert np.array_equal(got[count].view(np.uint32), got[rows][:count].view(np.uint32)), count
+    n = pool_elements(cfg, 16, 1)
+    keys, values = np.zeros(n, np.float32), np.zeros(n, np.float32)
+    table = np.zeros(1, dtype=np.int32)
+    model.append(keys, values, 16, table, 0, tokens[32:33])
+    want = model.append(keys, values, 16, table, 1, tokens[rows + 32:rows + 33])
+    assert rel_inf(got[rows][32], want) <= 1e-3
+
+
 def test_fast_small_batch_decode_gemv(torch_cuda):
     """Decode steps of up to four sequences take the GEMV projections
     (row-major weights, RMSNorm computed inside the projections): 90

@@ -671,11 +671,7 @@ hipError_t launch_fast(hipStream_t s, const FastGemmArgs& a) {
 // its two weight matrices make its column blocks the heaviest; up to 32 rows one,
 // 6.3-6.5 instead of 8.0-8.7 us at 1 and 32 rows). With many rows a tile of
 // 64 rows and 32 columns (two column blocks, of SwiGLU both matrices), or of
-// 64 x 16 where those are too few, reads weights and activations less often.
-// Either is taken from 7 work-groups per 4 CUs on: below, the wider tile
-// leaves CUs idle (SwiGLU of 512 rows, 384 tiles of 64 x 32: 28.5 vs 24.0 us
-// for 64 x 16; down at 512 rows, 288 of 64 x 16: 21.9 vs 20.0 for 16 x 16).
-// Such tiles take their steps one at a time (CH = 1): what hides their loads
+// 64 x 16 where those are too few (fast_large_tiles). Such tiles take their steps one at a time (CH = 1): what hides their loads
 // is a second and third work-group on the CU, which the registers of longer
 // chunks kept out. us at 4,096 rows with CH = 2 and 64 x 64 before: gate/up
 // 189 -> 155, q|k|v 80 -> 68, O and down 186 -> 158 together; at 512 rows 31
@@ -685,11 +681,9 @@ hipError_t launch_fast(hipStream_t s, const FastGemmArgs& a) {
 // again past the L2 (gate/up 50 vs 47 us at 1,000 rows, 20.0 vs 18.4 at 256).
 // Decode tiles keep them (64 rows: q|k|v 6.3 vs 6.9 us, a whole step of the
 // 30-layer model 1.0% less).
-constexpr int kCus = 256;
+constexpr int kCus = kChipCus;
 bool head_wide(int columns) { return columns % 64 == 0; }
 int tiles(const FastGemmArgs& a, int rb, int cb) { return ((a.rows + 15) / 16 + rb - 1) / rb * (a.columns / 16 / cb); }
-
-bool many(int tiles) { return 4 * tiles >= 7 * kCus; }
 
 template <int EPI, bool NORM, bool GATHER>
 hipError_t launch_sized(hipStream_t s, const FastGemmArgs& a) {
@@ -722,8 +716,8 @@ hipError_t launch_sized(hipStream_t s, const FastGemmArgs& a) {
         }
         return launch_fast<EPI, NORM, GATHER, 1, 1, 6>(s, a);
     } else {
-        if (a.columns % 32 == 0 && many(tiles(a, 4, 2))) return launch_fast<EPI, NORM, GATHER, 4, 2, 1>(s, a);
-        if (many(tiles(a, 4, 1))) return launch_fast<EPI, NORM, GATHER, 4, 1, 1>(s, a);
+        if (fast_large_tiles(a.rows, a.columns, 4, 2)) return launch_fast<EPI, NORM, GATHER, 4, 2, 1>(s, a);
+        if (fast_large_tiles(a.rows, a.columns, 4, 1)) return launch_fast<EPI, NORM, GATHER, 4, 1, 1>(s, a);
         if constexpr (EPI == kSwiglu) {
             if (a.rows > 64) return launch_fast<EPI, NORM, GATHER, 2, 1, 3>(s, a);
             if (a.rows > 32) return launch_fast<EPI, NORM, GATHER, 2, 1, 6>(s, a);
