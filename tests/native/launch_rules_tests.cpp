@@ -47,9 +47,21 @@ static void large_tiles() {
     CHECK(fast_large_tiles(2147483647 - 15, 1 << 20, 4, 2));
 }
 
+// A head whose weights outgrow the caches is streamed while one group of rows
+// reads it.
+static void head_streams() {
+    CHECK(fast_head_streams(1, 1024, 128256) && fast_head_streams(64, 1024, 128256));
+    CHECK(!fast_head_streams(65, 1024, 128256));
+    CHECK(fast_head_streams(16, 2048, 32000));
+    CHECK(!fast_head_streams(16, 512, 32768) && !fast_head_streams(1, 4096, 4096));
+    CHECK(!fast_head_streams(1, 1024, 32768) && fast_head_streams(1, 1024, 32832));
+    CHECK(fast_head_streams(1, 16384, 262144));
+}
+
 int main() {
     scores_in_global_memory();
     large_tiles();
+    head_streams();
     std::puts("ok");
     return 0;
 }

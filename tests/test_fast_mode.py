@@ -379,6 +379,37 @@ def test_fast_head_rows_do_not_depend_on_the_passes(torch_cuda, count, vocabular
     assert np.array_equal(together.view(np.uint32), apart.view(np.uint32))
 
 
+@pytest.mark.parametrize("vocabulary", [512, 32832])
+def test_fast_tiled_head_rows_same_in_any_tile(torch_cuda, vocabulary):
+    """The tiled LM head (hidden sizes other than 576) takes 16, 32 or 64 rows
+    a tile and streams its weights where they are large and one row group
+    reads them: 65 sequences decoded together, and 64, 32 and 7 of them, give
+    the same logits, bit for bit, within 1e-3 relative of the oracle, each
+    row's token its own first maximum."""
+    cfg = dict(layers=1, hidden=1024, intermediate=64, heads=16, kv_heads=4, vocabulary=vocabulary, context=32, eos=0,
+               rms_epsilon=1e-5, rope_theta=100000.0, tied=1)
+    model = OracleModel(cfg, seed=83)
+    o = Oracle()
+    rows = 65
+    tokens = [int(t) for t in o.fill_tokens(rows, 83, 9910, vocabulary)]
+    backend = HipBackend(cfg, block_tokens=16, max_blocks=rows, max_sequences=rows, arithmetic=ARITHMETIC_FAST)
+    upload_model(backend, model)
+    for i in range(rows):
+        backend.table_write(i, 0, np.array([i], dtype=np.int32))
+    got = {}
+    for count in (rows, 64, 32, 7):
+        am, logits = backend.forward([(i, 0, 1) for i in range(count)], tokens[:count])
+        assert all(a == int(np.argmax(g)) for a, g in zip(am, logits))
+        got[count] = logits.copy()
+    backend.close()
+    for count in (64, 32, 7):
+        assert np.array_equal(got[count].view(np.uint32), got[rows][:count].view(np.uint32)), count
+    n = pool_elements(cfg, 16, 1)
+    keys, values = np.zeros(n, np.float32), np.zeros(n, np.float32)
+    want = model.append(keys, values, 16, np.zeros(1, dtype=np.int32), 0, tokens[64:])
+    assert rel_inf(got[rows][64], want) <= 1e-3
+
+
 @pytest.mark.parametrize("intermediate", [7168, 14336])
 def test_fast_wide_projection_rows_same_in_any_tile(torch_cuda, intermediate):
     """Wide projections take 16-row tiles up to 32 rows and 64-row tiles of one

@@ -102,7 +102,7 @@ __device__ __forceinline__ uint64_t max_key(uint64_t key) {
 __device__ __forceinline__ int rope_dim(int cb, int lane) { return fast_rope_column(cb * 16 + (lane & 15)) & 63; }
 __device__ __forceinline__ int rope_pair(int cb, int lane) { return 8 * (cb & 3) + (lane & 7); }
 
-template <int EPI, bool NORM, bool GATHER, int RB, int CB, int CH>
+template <int EPI, bool NORM, bool GATHER, int RB, int CB, int CH, bool STREAM>
 __global__ __launch_bounds__(kWaves * 64, CH == 1 ? 4 : 1) void fast_gemm_kernel(FastGemmArgs a) {
     constexpr int M = EPI == kSwiglu ? 2 : 1;
     constexpr int NB = CB * M;  // B operands per step
@@ -112,9 +112,6 @@ __global__ __launch_bounds__(kWaves * 64, CH == 1 ? 4 : 1) void fast_gemm_kernel
     // barrier precedes the owners' sums; more tiles are summed in two levels
     // (wavefronts 4-7 into 0-3, then to the owners) to halve the LDS.
     constexpr bool kOneSync = T <= 4;
-    // Decode tiles (long chunks) stream their weights; launch_sized says why
-    // the others do not.
-    constexpr bool kStreamWeights = CH >= 6;
     __shared__ f4 part_s[kOneSync ? kWaves : kWaves / 2][T][64];
     __shared__ float ssq_s[NORM ? RB * 16 : 1][kSsqSlots];
     __shared__ float inv_s[RB * 16];
@@ -225,7 +222,7 @@ __global__ __launch_bounds__(kWaves * 64, CH == 1 ? 4 : 1) void fast_gemm_kernel
 #pragma unroll
                 for (int j = 0; j < NB; ++j) {
                     const f4* w4 = reinterpret_cast<const f4*>(wb[j] + s * 256);
-                    bv[c][j] = kStreamWeights ? __builtin_nontemporal_load(w4) : *w4;
+                    bv[c][j] = STREAM ? __builtin_nontemporal_load(w4) : *w4;
                 }
             }
         }
@@ -656,13 +653,14 @@ __global__ __launch_bounds__(256) void fast_ssq_kernel(const float* __restrict__
     ssq[(size_t)p * stride + r] = s;
 }
 
-template <int EPI, bool NORM, bool GATHER, int RB, int CB, int CH>
+// STREAM: nontemporal weight loads (launch_sized says where).
+template <int EPI, bool NORM, bool GATHER, int RB, int CB, int CH, bool STREAM = CH >= 6>
 hipError_t launch_fast(hipStream_t s, const FastGemmArgs& a) {
     const int nrg = ((a.rows + 15) / 16 + RB - 1) / RB;
     const int ncg = a.columns / 16 / CB;
     const int blocks = a.rows > kSpreadRows ? (nrg * ncg + kXcds - 1) / kXcds * kXcds
                                             : (ncg + kXcds - 1) / kXcds * nrg * kXcds;
-    fast_gemm_kernel<EPI, NORM, GATHER, RB, CB, CH><<<blocks, kWaves * 64, 0, s>>>(a);
+    fast_gemm_kernel<EPI, NORM, GATHER, RB, CB, CH, STREAM><<<blocks, kWaves * 64, 0, s>>>(a);
     return hipGetLastError();
 }
 
@@ -671,16 +669,18 @@ hipError_t launch_fast(hipStream_t s, const FastGemmArgs& a) {
 // its two weight matrices make its column blocks the heaviest; up to 32 rows one,
 // 6.3-6.5 instead of 8.0-8.7 us at 1 and 32 rows). With many rows a tile of
 // 64 rows and 32 columns (two column blocks, of SwiGLU both matrices), or of
-// 64 x 16 where those are too few (fast_large_tiles). Such tiles take their steps one at a time (CH = 1): what hides their loads
-// is a second and third work-group on the CU, which the registers of longer
-// chunks kept out. us at 4,096 rows with CH = 2 and 64 x 64 before: gate/up
-// 189 -> 155, q|k|v 80 -> 68, O and down 186 -> 158 together; at 512 rows 31
-// -> 24, 16 -> 12.6, 43 -> 30; at 256 rows gate/up (two row blocks, CH = 3
-// instead of 6) 19.4 -> 17.0 and q|k|v 11.6 -> 8.9. From 65 rows on the weights
-// are read with plain loads: nontemporal ones made each row group fetch them
+// 64 x 16 where those are too few (fast_large_tiles). Such tiles take their
+// steps one at a time (CH = 1): what hides their loads is a second work-group
+// on the CU (a third for 64 x 16), which the registers of longer chunks kept
+// out. us at 4,096 rows with CH = 2 and 64 x 64 before: gate/up 189 -> 155,
+// q|k|v 80 -> 68, O and down 186 -> 158 together; at 512 rows 31 -> 24, 16 ->
+// 12.6, 43 -> 30; at 256 rows gate/up (two row blocks, CH = 3 instead of 6)
+// 19.4 -> 17.0 and q|k|v 11.6 -> 8.9. The tiles of one or three steps read the
+// weights with plain loads: nontemporal ones made each row group fetch them
 // again past the L2 (gate/up 50 vs 47 us at 1,000 rows, 20.0 vs 18.4 at 256).
-// Decode tiles keep them (64 rows: q|k|v 6.3 vs 6.9 us, a whole step of the
-// 30-layer model 1.0% less).
+// The longer chunks (up to 64 rows; O, down and few-column q|k|v up to 256)
+// stream them (64 rows: q|k|v 6.3 vs 6.9 us, a whole step of the 30-layer
+// model 1.0% less).
 constexpr int kCus = kChipCus;
 bool head_wide(int columns) { return columns % 64 == 0; }
 int tiles(const FastGemmArgs& a, int rb, int cb) { return ((a.rows + 15) / 16 + rb - 1) / rb * (a.columns / 16 / cb); }
@@ -708,11 +708,15 @@ hipError_t launch_sized(hipStream_t s, const FastGemmArgs& a) {
             return hipGetLastError();
         }
         if (head_wide(a.columns)) {
-            // Row blocks as the batch needs them (B=1: 24.6 instead of 52.4
-            // us; B=32: 35.0 instead of 48.6), 64-column groups throughout.
-            if (a.rows <= 16) return launch_fast<EPI, NORM, GATHER, 1, 4, 1>(s, a);
-            if (a.rows <= 32) return launch_fast<EPI, NORM, GATHER, 2, 4, 1>(s, a);
-            return launch_fast<EPI, NORM, GATHER, 4, 4, 1>(s, a);
+            // Row blocks as the batch needs them (49,152 columns of hidden size
+            // 576, before it had the kernel above: one row 24.6 instead of 52.4
+            // us, 32 rows 35.0 instead of 48.6), 64-column groups throughout.
+            const bool stream = fast_head_streams(a.rows, a.inner, a.columns);
+            if (a.rows <= 16)
+                return stream ? launch_fast<EPI, NORM, GATHER, 1, 4, 1, true>(s, a) : launch_fast<EPI, NORM, GATHER, 1, 4, 1>(s, a);
+            if (a.rows <= 32)
+                return stream ? launch_fast<EPI, NORM, GATHER, 2, 4, 1, true>(s, a) : launch_fast<EPI, NORM, GATHER, 2, 4, 1>(s, a);
+            return stream ? launch_fast<EPI, NORM, GATHER, 4, 4, 1, true>(s, a) : launch_fast<EPI, NORM, GATHER, 4, 4, 1>(s, a);
         }
         return launch_fast<EPI, NORM, GATHER, 1, 1, 6>(s, a);
     } else {

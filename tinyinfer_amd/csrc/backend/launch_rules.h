@@ -31,4 +31,16 @@ constexpr bool fast_large_tiles(int rows, int columns, int row_blocks, int colum
     return 4 * tiles >= 7 * kChipCus;
 }
 
+// Whether the tiled LM head (hidden sizes other than 576) streams its weights
+// past the caches: where one group of up to 64 rows reads them and they would
+// not stay in the last-level cache (256 MiB) beside the rest of the model.
+// Streamed against plain loads at 1 to 16 rows: 98 vs 110 us for 525 MB
+// (hidden 1,024, 128,256 columns), 54.5 vs 58 for 262 MB (2,048, 32,000; in a
+// model of 8 layers), but 46 vs 46 for 67 MB (4,096, 4,096; 4 layers) and 21
+// vs 20 (512, 32,768; 16 layers). Two row groups share plain loads' lines:
+// 331 vs 323 us at 65 rows of the first, 57 vs 53 of the last.
+constexpr bool fast_head_streams(int rows, int inner, int columns) {
+    return rows <= 64 && (long long)inner * columns > 32ll << 20;  // floats: 128 MiB
+}
+
 }  // namespace mphip
