@@ -58,10 +58,23 @@ static void head_streams() {
     CHECK(fast_head_streams(1, 16384, 262144));
 }
 
+static void head_columns() {
+    for (int rows : {1, 64, 200})
+        for (int columns : {4, 4096, 49152}) CHECK(exact_head_columns(576, columns, rows) == 16);
+    CHECK(exact_head_columns(608, 49152, 1) == 64 && exact_head_columns(2020, 32000, 256) == 64);
+    CHECK(exact_head_columns(608, 4096, 128) == 16 && exact_head_columns(608, 4096, 129) == 64);
+    CHECK(exact_head_columns(608, 8192, 64) == 16 && exact_head_columns(608, 8196, 64) == 64);
+    CHECK(exact_head_groups(576, 49152, 1) == 3072 && exact_head_groups(608, 49152, 1) == 768);
+    CHECK(exact_head_groups(576, 4, 1) == 1 && exact_head_groups(576, 20, 1) == 2);
+    CHECK(exact_head_groups(608, 8260, 64) == 130);
+    CHECK(exact_head_columns(4, 2147483647 - 63, 2147483647 - 63) == 64);
+}
+
 int main() {
     scores_in_global_memory();
     large_tiles();
     head_streams();
+    head_columns();
     std::puts("ok");
     return 0;
 }

@@ -139,6 +139,31 @@ def test_prefill_projection_shapes(torch_cuda, hidden, intermediate, vocabulary,
     _run_sequence(model, backend, 16, [prompt[:3], prompt[3:], prompt[:1]], table)
 
 
+@pytest.mark.parametrize("hidden,vocabulary", [(80, 60), (80, 200), (80, 8260), (128, 200)])
+def test_head_of_any_hidden_size(torch_cuda, hidden, vocabulary):
+    """The LM head with rows of weights that are whole 64-wide chunks (128) and
+    that are not (80: 16 columns a work-group, or 64 for 8,260), with columns
+    in a last, partly empty group: 66 sequences decoded together give each its
+    own logits and first maximum, bit for bit."""
+    cfg = tiny_config(hidden=hidden, intermediate=64, heads=hidden // 16, kv_heads=hidden // 16, vocabulary=vocabulary,
+                      context=32, tied=1)
+    model = OracleModel(cfg, seed=43, stddev=0.05)
+    rows = 66
+    backend = HipBackend(cfg, block_tokens=16, max_blocks=rows, max_sequences=rows)
+    upload_model(backend, model)
+    for i in range(rows):
+        backend.table_write(i, 0, np.array([i], dtype=np.int32))
+    tokens = [int(t) for t in Oracle().fill_tokens(rows, 43, 3500, vocabulary)]
+    am, got = backend.forward([(i, 0, 1) for i in range(rows)], tokens)
+    backend.close()
+    n = pool_elements(cfg, 16, 1)
+    for i in range(rows):
+        keys, values = np.zeros(n, np.float32), np.zeros(n, np.float32)
+        want = model.append(keys, values, 16, np.zeros(1, dtype=np.int32), 0, tokens[i:i + 1])
+        assert np.array_equal(got[i].view(np.uint32), want.view(np.uint32)), i
+        assert am[i] == int(np.argmax(want)), i
+
+
 @pytest.mark.parametrize("group", [1, 4])
 def test_prefill_scores_of_other_groups(torch_cuda, group):
     """64-wide heads with 1 and 4 query heads per KV head: the row blocks'

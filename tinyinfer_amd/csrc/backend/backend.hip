@@ -333,8 +333,8 @@ int ensure_workspace(mp_hip* h, int rows, int seqs, int max_length) {
     h->row_rope = h->fast_partials = nullptr;
     h->workspace_rows = h->workspace_seqs = 0;
     const size_t hd = c.hidden;
-    const size_t groups = h->fast ? std::max<size_t>(mphip::head_groups(c.vocabulary), c.vocabulary / 16)
-                                  : mphip::head_groups(c.vocabulary);
+    static_assert(mphip::kExactHeadColumns == 16, "the fast head's narrowest groups, too");
+    const size_t groups = ((size_t)c.vocabulary + 15) / 16;
     struct Item { void** p; size_t bytes; };
     const Item items[] = {
         {(void**)&h->x, sizeof(float) * R * hd},
@@ -1358,7 +1358,7 @@ int mp_hip_forward(mp_hip* h, const mp_seq_step* steps, int32_t nseq, const int3
         a.best_value = h->best_value;
         a.best_index = h->best_index;
         a.bad = h->best_bad;
-        a.groups = mphip::head_groups(c.vocabulary);
+        a.groups = mphip::exact_head_groups(hd, c.vocabulary, nseq);
         if (r == hipSuccess) r = mphip::launch_gemm(s, mphip::kHead, a);
         if (r == hipSuccess) r = mphip::launch_head_argmax(s, a, h->results, h->results + nseq);
         return r;

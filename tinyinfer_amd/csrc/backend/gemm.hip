@@ -957,7 +957,6 @@ hipError_t launch_column_one(hipStream_t s, const GemmArgs& a) {
 
 }  // namespace
 
-int head_groups(int columns) { return (columns + kHeadColumns - 1) / kHeadColumns; }
 
 bool gemm_normed_fits(Epilogue epilogue, const GemmArgs& a) {
     return a.rows > 0 && a.rows <= 64 && a.columns > 0 && a.inner > 0 && a.inner % 64 == 0 &&
@@ -1005,9 +1004,12 @@ hipError_t launch_gemm(hipStream_t s, Epilogue epilogue, const GemmArgs& a) {
     case kResidual: return many ? launch_shape<4, 4, kResidual, 5>(s, a) : launch_shape<1, 4, kResidual, 6>(s, a);
     case kSwiglu: return many ? launch_shape<4, 4, kSwiglu, 5>(s, a) : launch_shape<1, 4, kSwiglu, 6>(s, a);
     case kHead:
-        static_assert(8 * kScalarColumns == kHeadColumns, "head work-group width");
+        if (a.groups != exact_head_groups(a.inner, a.columns, a.rows)) return hipErrorInvalidValue;
+        static_assert(8 * kScalarColumns == kExactHeadColumns, "head work-group width");
         if (a.inner % kChunk == 0) return launch_scalar<8, kHead>(s, a);
-        return launch_shape<kScalarColumns, 8, kHead, 4>(s, a);
+        return exact_head_columns(a.inner, a.columns, a.rows) == kExactHeadColumns
+                   ? launch_shape<kScalarColumns, 8, kHead, 4>(s, a)
+                   : launch_shape<8, 8, kHead, 4>(s, a);
     }
     return hipErrorInvalidValue;
 }

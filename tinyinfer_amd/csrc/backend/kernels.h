@@ -39,7 +39,7 @@ enum Epilogue { kStore = 0, kResidual = 1, kSwiglu = 2, kHead = 3, kRope = 4 };
 // layout), w is [columns][inner]. kStore writes out (quad layout, `columns`
 // wide); kResidual adds into out; kSwiglu computes (g/(1+exp(-g)))*u from the
 // chains of w (g) and w2 (u); kHead writes, per row and per group of
-// kHeadColumns columns, the first maximum and a non-finite flag into the
+// exact_head_columns(inner, columns, rows) columns, the first maximum and a non-finite flag into the
 // partial arrays, and the logits row-major into `out` when it is non-null.
 struct GemmArgs {
     const float* x;
@@ -56,8 +56,6 @@ struct GemmArgs {
     int32_t* bad;
     int groups;
 };
-constexpr int kHeadColumns = 16;
-int head_groups(int columns);
 hipError_t launch_gemm(hipStream_t s, Epilogue epilogue, const GemmArgs& args);
 // The same projection of RMSNorm(x) (llama_runner.cpp:10-16 then :30-36)
 // in one launch where the shape allows (one row tile, inner <= 576 and a

@@ -43,4 +43,21 @@ constexpr bool fast_head_streams(int rows, int inner, int columns) {
     return rows <= 64 && (long long)inner * columns > 32ll << 20;  // floats: 128 MiB
 }
 
+// Columns of the exact LM head per work-group (and per argmax partial): 8
+// wavefronts of two columns, their weights as scalars, where a row of weights
+// is whole 64-wide chunks. Elsewhere the weights go through LDS and eight
+// columns share an x read: 128 instead of 203 us for 49,152 columns of hidden
+// size 608 at 1 to 64 rows, 54 instead of 78 for 4,096 columns at 200 rows;
+// two columns where eight leave half the chip idle (4,096 columns: 31 instead
+// of 51 us up to 64 rows, 48 instead of 53 up to 128).
+constexpr int kExactHeadColumns = 16;  // the fewest
+constexpr int exact_head_columns(int inner, int columns, int rows) {
+    const long long wide = (long long)((columns + 63) / 64) * ((rows + 63) / 64);
+    return inner % 64 && 2 * wide > kChipCus ? 64 : kExactHeadColumns;
+}
+constexpr int exact_head_groups(int inner, int columns, int rows) {
+    const int group = exact_head_columns(inner, columns, rows);
+    return (columns + group - 1) / group;
+}
+
 }  // namespace mphip
