@@ -70,11 +70,24 @@ static void head_columns() {
     CHECK(exact_head_columns(4, 2147483647 - 63, 2147483647 - 63) == 64);
 }
 
+// Long rows take their heads apart in the kernel for 16-token pages and
+// 64-wide heads only, few rows in every kernel.
+static void heads_apart() {
+    for (int group = 1; group <= 8; ++group) {
+        CHECK(exact_heads_apart(512, group, 64, true) && exact_heads_apart(1, group, 40000, true));
+        CHECK(!exact_heads_apart(513, group, 1024, true) && exact_heads_apart(513, group, 1025, true));
+        CHECK(exact_heads_apart(1, group, 40000, false) && exact_heads_apart(256, group, 64, false));
+        CHECK(!exact_heads_apart(513, group, 1025, false) && !exact_heads_apart(1ll << 40, group, 32768, false));
+    }
+    CHECK(!exact_heads_apart(257, 3, 1000, false) && exact_heads_apart(512, 4, 1000, false));
+}
+
 int main() {
     scores_in_global_memory();
     large_tiles();
     head_streams();
     head_columns();
+    heads_apart();
     std::puts("ok");
     return 0;
 }

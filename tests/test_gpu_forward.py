@@ -180,6 +180,22 @@ def test_prefill_scores_of_other_groups(torch_cuda, group):
     _run_sequence(model, backend, 16, [prompt[:2], prompt[2:35], prompt[35:240], prompt[240:283], prompt[:1]], table)
 
 
+@pytest.mark.parametrize("dim,group,bt", [(32, 2, 16), (32, 3, 16), (48, 4, 16), (64, 3, 32), (64, 3, 16)])
+def test_prefill_softmax_heads_apart_and_together(torch_cuda, dim, group, bt):
+    """The softmax and output of a KV head's query heads run apart for few
+    rows (30) and together for many (300, in rows past 1,024 tokens too; apart
+    there with 16-token pages and 64-wide heads), bit for bit."""
+    cfg = tiny_config(hidden=dim * group, intermediate=64, heads=group, kv_heads=1, vocabulary=128, context=1280, tied=1)
+    model = OracleModel(cfg, seed=47, stddev=0.08)
+    blocks = 1280 // bt
+    backend = HipBackend(cfg, block_tokens=bt, max_blocks=blocks, max_sequences=1)
+    upload_model(backend, model)
+    o = Oracle()
+    prompt = [int(t) for t in o.fill_tokens(1231, 47, 3600, 128)]
+    table = o.permutation(blocks, 47, 3601).copy()
+    _run_sequence(model, backend, bt, [prompt[:300], prompt[300:900], prompt[900:1200], prompt[1200:1230], prompt[:1]], table)
+
+
 def test_batched_rows_match_single_sequences(torch_cuda):
     """Several sequences in one forward call == each appended alone."""
     cfg = smollm_config(layers=2, context=256)

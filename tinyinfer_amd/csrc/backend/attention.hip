@@ -909,8 +909,6 @@ hipError_t launch_fused_decode(hipStream_t s, const float* qkv, int ldq, int hea
     return hipGetLastError();
 }
 
-constexpr int kPvApartTasks = 512, kPvApartLength = 1024;
-
 template <int BT, int DIM>
 hipError_t launch_pair(hipStream_t s, const float* qkv, int ldq, int heads, int kv_heads, int dim,
                        const RowMeta& meta, const PagedKv& kv, int layer, float* out, int ldo,
@@ -928,12 +926,8 @@ hipError_t launch_pair(hipStream_t s, const float* qkv, int ldq, int heads, int 
         launch_timed(attn_pv_kernel<BT, DIM, 1>, dim3(w.blocks_count, kv_heads, group), wg, s, nullptr, ev.stop, heads,
                      kv_heads, dim, meta, kv, layer, w, out, ldo);
     } else {
-        // A wavefront per query head (its own e_t and chain, V read once per
-        // head) where few rows leave SIMDs idle or rows are long, else one for
-        // the KV head's heads. Apart against together: 7.5 vs 12.4 us for 30
-        // rows at position 100, 127 vs 134 for 256 rows at 3,000 and 128 vs
-        // 135 for 1,024 at 1,000, but 25.5 vs 24.2 for 256 at 256.
-        const bool apart = w.blocks_count * kv_heads * block_rows <= kPvApartTasks || w.stride > kPvApartLength;
+        const bool apart = exact_heads_apart((long long)w.blocks_count * kv_heads * block_rows, group, w.stride,
+                                             BT == 16 && DIM == 64);
         const dim3 grid(w.blocks_count, kv_heads, block_rows);
         switch (apart ? 1 : group) {
         case 2: launch_timed(attn_pv_kernel<BT, DIM, 2>, grid, wg, s, nullptr, ev.stop, heads, kv_heads, dim, meta, kv, layer, w, out, ldo); break;

@@ -60,4 +60,21 @@ constexpr int exact_head_groups(int inner, int columns, int rows) {
     return (columns + group - 1) / group;
 }
 
+// Whether the exact prefill attention computes a row's softmax and output one
+// query head a wavefront (its own e_t and chain, V read once per head) or a KV
+// head's together: apart where few tasks (rows times KV heads) leave SIMDs
+// idle, and in the kernel for 16-token pages and 64-wide heads for long rows
+// as well. `longest` is the step's longest row. Apart against together, us:
+// 7.5 vs 12.4 for 30 rows at position 100, 127 vs 134 for 256 rows at 3,000
+// and 128 vs 135 for 1,024 at 1,000, but 25.5 vs 24.2 for 256 at 256. The
+// kernel for other shapes is bound by its scattered V reads, which apart it
+// makes once per head: three heads of 48 dims, 256 rows, 508 vs 292 at 1,000
+// and 1,283 vs 730 at 3,000; two of 32 dims 571 vs 493 and 1,478 vs 1,300;
+// three of 32, 100 rows (448 tasks) 244 vs 217 at 1,000 but 30 rows (128) 178
+// vs 187; four of 32 gain with 100 rows as well (246 vs 295).
+constexpr bool exact_heads_apart(long long tasks, int group, int longest, bool paged16x64) {
+    if (paged16x64) return tasks <= 512 || longest > 1024;
+    return tasks <= (group > 3 ? 512 : 256);
+}
+
 }  // namespace mphip
