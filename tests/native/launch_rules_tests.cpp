@@ -82,8 +82,32 @@ static void heads_apart() {
     CHECK(!exact_heads_apart(257, 3, 1000, false) && exact_heads_apart(512, 4, 1000, false));
 }
 
+// The row kernel at the measured sizes that are clear either way, and that it
+// stays once a row is long enough.
+static void row_kernel() {
+    CHECK(attention_row_pays(9, 3, 1) && attention_row_pays(9, 3, 503) && attention_row_pays(32, 4, 1));
+    CHECK(!attention_row_pays(32, 32, 64) && attention_row_pays(32, 32, 128));
+    CHECK(!attention_row_pays(128, 128, 64) && !attention_row_pays(128, 128, 256) && attention_row_pays(128, 128, 1000));
+    CHECK(!attention_row_pays(128, 32, 64) && attention_row_pays(128, 32, 256) && attention_row_pays(128, 16, 1));
+    CHECK(!attention_row_pays(192, 192, 1000) && attention_row_pays(192, 192, 8192));
+    CHECK(!attention_row_pays(256, 256, 8192) && !attention_row_pays(384, 384, 10240));
+    CHECK(!attention_row_pays(256, 32, 100) && attention_row_pays(256, 32, 300));
+    for (int group = 1; group <= 8; ++group)
+        for (int kv_heads : {1, 3, 16}) {
+            bool before = false;
+            for (int length = 1; length <= 10240; ++length) {
+                const bool now = attention_row_pays(group * kv_heads, kv_heads, length);
+                CHECK(now || !before || length <= 32);
+                before = now;
+            }
+            CHECK(before);
+        }
+    CHECK(!attention_row_pays(1 << 20, 1 << 20, 10240));
+}
+
 int main() {
     scores_in_global_memory();
+    row_kernel();
     large_tiles();
     head_streams();
     head_columns();

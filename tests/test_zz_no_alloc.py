@@ -105,6 +105,15 @@ def test_row_kernel_groups(torch_cuda, group):
         _check(torch_cuda, Oracle(), 200 + group, length, 2 * group, 2)
 
 
+@pytest.mark.parametrize("heads,kv_heads", [(16, 16), (72, 24), (128, 128)])
+def test_many_heads(torch_cuda, heads, kv_heads):
+    """Short rows of heads of their own and rows of very many heads take the
+    general kernel, longer ones the row kernel: bits of the oracle on both
+    sides."""
+    for length in (1, 63, 90, 130, 600, 1000):
+        _check(torch_cuda, Oracle(), 350, length, heads, kv_heads)
+
+
 @pytest.mark.parametrize("scale,equal", [(0.0, False), (1.0, True), (8.0, False), (0.05, False)])
 def test_row_kernel_denominators(torch_cuda, scale, equal):
     """Denominators that are exact in every step (equal scores: all e_t are

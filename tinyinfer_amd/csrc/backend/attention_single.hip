@@ -10,7 +10,8 @@
 // order is kept by ordered_sum.h with a whole wavefront.)
 //
 // Pages of 16 tokens with 64-wide heads take the kernels at the end of this
-// file; other shapes the general kernel below.
+// file (except where attention_row_pays says otherwise, and where out lies
+// over q); other shapes the general kernel below.
 #include "exact_math.h"
 #include "kernels.h"
 #include "layout.h"
@@ -579,7 +580,8 @@ hipError_t launch_attention_single(hipStream_t s, const float* q, const float* k
     // work-group touches them: such calls take it.
     const size_t width = (size_t)heads * dim;
     const bool over_q = (uintptr_t)out < (uintptr_t)(q + width) && (uintptr_t)q < (uintptr_t)(out + width);
-    if (block_tokens == kRowPage && dim == kRowDim && (scratch || (length <= kRowWindow && !over_q))) {
+    if (block_tokens == kRowPage && dim == kRowDim &&
+        (scratch || (length <= kRowWindow && !over_q && attention_row_pays(heads, kv_heads, length)))) {
         const RowArgs a{q, keys, values, table, length, layer, layers, heads, kv_heads, out, scratch};
         switch (heads / kv_heads) {
         case 1: launch_row<1>(s, a); break;

@@ -6,11 +6,31 @@
 
 namespace mphip {
 
+constexpr int kChipCus = 256;
+
 // Score floats of a KV head's query heads that the stand-alone single-row
 // attention keeps on the chip; longer rows take theirs through global memory.
 constexpr int kAttentionLdsScores = 10240;
 constexpr bool attention_scores_global(int group, int length) {
     return (size_t)group * (((size_t)length + 15) & ~(size_t)15) > (size_t)kAttentionLdsScores;
+}
+
+// Whether a single-row attention with 16-token pages and 64-wide heads whose
+// scores stay on the chip takes the row kernel: four work-groups of a whole CU
+// for each query head, against one work-group for a KV head's heads whose
+// output chains take three times as long. The row kernel loses where a row is
+// short, and where many heads make it take several turns of the chip. Both
+// estimates are in ns, fitted over 1 to 384 heads, 1 to 8 of them per KV head,
+// and 1 to 8,192 tokens (general and row kernel, us): 32 heads apart 9.3 and
+// 10.6 at 64 tokens, 13 and 11.6 at 128, 36 and 19 at 503; 128 apart 9.4 and
+// 20 at 64, 38 and 42 at 503, 77 and 66 at 1,000, 149 and 104 at 2,000; 256
+// apart 43 and 81 at 503, 707 and 746 at 8,192; 256 on 32 KV heads 39 and 42
+// at 128, 50 and 49 at 200, 102 and 71 at 503.
+constexpr bool attention_row_pays(int heads, int kv_heads, int length) {
+    const long long group = heads / kv_heads, turns = (4ll * heads + kChipCus - 1) / kChipCus;
+    const long long general = 3500 + 2900 * group + (67 * ((group + 3) / 4) + 5 * group) * (length > 32 ? length - 32 : 0);
+    const long long row = 1000 + turns * (9300 + (turns == 1 ? 14ll : 16 + 6 / group) * length);
+    return row < general;
 }
 
 // Whether a fast projection of `rows` x `columns` takes tiles of `row_blocks`
@@ -24,7 +44,7 @@ constexpr bool attention_scores_global(int group, int length) {
 // to 14,336 columns) with 64-row tiles against 16-row ones: 310 to 580 vs 260
 // to 408 us at 1 to 16 rows, 312 to 593 vs 303 to 561 at 17, the same at 32,
 // 350 to 700 vs 377 to 820 at 33.
-constexpr int kChipCus = 256, kLargeTileRows = 33;
+constexpr int kLargeTileRows = 33;
 constexpr bool fast_large_tiles(int rows, int columns, int row_blocks, int column_blocks) {
     if (rows < kLargeTileRows || columns % (16 * column_blocks)) return false;
     const long long tiles = (long long)(((rows + 15) / 16 + row_blocks - 1) / row_blocks) * (columns / 16 / column_blocks);
