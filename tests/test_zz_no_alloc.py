@@ -169,3 +169,31 @@ def test_rows_with_scores_on_the_chip_may_overlap(torch_cuda):
         torch.cuda.synchronize()
         for length, _, want, out, _ in rows:
             assert np.array_equal(out.cpu().numpy().view(np.uint32), want.view(np.uint32)), length
+
+
+@pytest.mark.parametrize("length", [300, 1500, 5000])
+def test_row_kernel_infinities_and_nans(torch_cuda, length):
+    """Infinite and NaN keys (either sign, in the first 256 tokens and in the
+    last ones) and values: the oracle's bits where it is not NaN, NaN exactly
+    where it is. One KV head holds the odd values, the others stay finite."""
+    torch, o = torch_cuda, Oracle()
+    bad = [("keys", np.inf), ("keys", -np.inf), ("keys", np.nan), ("keys", -np.nan), ("values", np.inf),
+           ("values", np.nan)]
+    for i, (where, value) in enumerate(bad):
+        for token in (7, length - 3):
+            q, keys, values, table = _inputs(o, 600 + i, length)
+            pool = (keys if where == "keys" else values).reshape(-1, LAYERS, BT, KV_HEADS, DIM)
+            pool[table[token // BT], LAYER, token % BT, 1, 5] = value
+            with np.errstate(all="ignore"):
+                want = o.attention(q, keys, values, table, length - 1, 1, LAYER, LAYERS, BT, HEADS, KV_HEADS, DIM)[0]
+            dq, dk, dv, dt = (torch.from_numpy(a).cuda() for a in (q, keys, values, table))
+            for call in (paged_attention_decode, paged_attention_decode_noalloc):
+                out = torch.zeros(HEADS * DIM, dtype=torch.float32, device="cuda")
+                call(dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dt.data_ptr(), length, LAYER, LAYERS, BT, HEADS,
+                     KV_HEADS, DIM, out.data_ptr(), None)
+                torch.cuda.synchronize()
+                got = out.cpu().numpy()
+                assert np.array_equal(np.isnan(got), np.isnan(want)), (where, value, token)
+                ok = ~np.isnan(want)
+                assert np.array_equal(got[ok].view(np.uint32), want[ok].view(np.uint32)), (where, value, token)
+                assert np.all(np.isfinite(np.delete(got.reshape(KV_HEADS, -1), 1, axis=0)))

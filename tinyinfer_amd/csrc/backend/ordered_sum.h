@@ -72,7 +72,7 @@ __device__ __forceinline__ float ordered_sum(const float* v, int n, float sum) {
     in_order(0, at);
     while (at < n4) {  // uniform: `sum` and `at` are the same in every lane
         const int bits = __builtin_amdgcn_readfirstlane(__float_as_int(sum));
-        const int exponent = bits >> 23;  // the sum is never negative
+        const int exponent = bits >> 23 & 255;  // the sum is never negative, but a NaN may have its sign set
         if (exponent == 0 || exponent >= 255) {
             const int to = exponent ? n4 : min(n4, at + kOrderedFirst / 4);
             in_order(at, to);
