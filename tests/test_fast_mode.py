@@ -266,6 +266,52 @@ def test_fast_prefill_chunking_does_not_change_rows(torch_cuda):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
+def test_fast_prefill_after_forks_and_rollbacks(torch_cuda):
+    """Prefill writes K and V in the projection's epilogue: a fork of a 40-token
+    prompt (two shared pages, the third copied at its 8 valid tokens) and the
+    prompt itself continue with different 21-token chunks in one step; then
+    the prompt is rolled back to 45 tokens and takes 33 others beside the
+    fork's next 18, and the fork decodes. The logits equal those of each text
+    run alone in a fresh context, bit for bit."""
+    cfg = smollm_config(layers=2, context=256, vocabulary=4096)
+    model = OracleModel(cfg, seed=89)
+    o = Oracle()
+    tokens = lambda n, stream: [int(t) for t in o.fill_tokens(n, 89, stream, cfg["vocabulary"])]
+    prompt, a, b, c, d = (tokens(n, 9920 + i) for i, n in enumerate((40, 21, 21, 33, 18)))
+    kvw = cfg["kv_heads"] * (cfg["hidden"] // cfg["heads"])
+    page, block = 16 * kvw, cfg["layers"] * 16 * kvw
+    backend = HipBackend(cfg, block_tokens=16, max_blocks=24, max_sequences=2, arithmetic=ARITHMETIC_FAST)
+    upload_model(backend, model)
+    backend.table_write(0, 0, np.array([20, 3, 11, 7, 1, 15], dtype=np.int32))
+    backend.forward([(0, 0, 40)], prompt)
+    backend.table_write(1, 0, np.array([20, 3, 9, 22, 5, 2], dtype=np.int32))
+    backend.copy_tail(9 * block, 11 * block, page, 8 * kvw, cfg["layers"])
+    _, first = backend.forward([(0, 40, 21), (1, 40, 21)], a + b)
+    _, second = backend.forward([(0, 45, 33), (1, 61, 18)], c + d)
+    _, third = backend.forward([(1, 79, 1)], [5])
+    backend.close()
+
+    def alone(text):
+        fresh = HipBackend(cfg, block_tokens=16, max_blocks=24, max_sequences=1, arithmetic=ARITHMETIC_FAST)
+        upload_model(fresh, model)
+        fresh.table_write(0, 0, np.arange(8, dtype=np.int32))
+        _, logits = fresh.forward([(0, 0, len(text))], text)
+        fresh.close()
+        return logits[0].view(np.uint32).copy()
+
+    assert np.array_equal(first[0].view(np.uint32), alone(prompt + a))
+    assert np.array_equal(first[1].view(np.uint32), alone(prompt + b))
+    assert np.array_equal(second[0].view(np.uint32), alone(prompt + a[:5] + c))
+    assert np.array_equal(second[1].view(np.uint32), alone(prompt + b + d))
+    fresh = HipBackend(cfg, block_tokens=16, max_blocks=24, max_sequences=1, arithmetic=ARITHMETIC_FAST)
+    upload_model(fresh, model)
+    fresh.table_write(0, 0, np.arange(8, dtype=np.int32))
+    fresh.forward([(0, 0, 79)], prompt + b + d)
+    _, want = fresh.forward([(0, 79, 1)], [5])
+    fresh.close()
+    assert np.array_equal(third.view(np.uint32), want.view(np.uint32))
+
+
 def test_fast_prefill_climbing_scores(torch_cuda):
     """Prefill rows whose scores climb by far more than the softmax's
     rescale margin of 16 across the pages a wavefront walks: 2,000 cached
