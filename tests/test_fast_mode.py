@@ -362,7 +362,8 @@ def test_fast_prefill_climbing_scores(torch_cuda):
 @pytest.mark.parametrize("group", [1, 2, 3, 4])
 def test_fast_prefill_rows_same_in_small_and_large_launches(torch_cuda, group):
     """The prefill attention computes a KV head's query heads in separate
-    work-groups up to 512 (16-row block, KV head) items and together beyond:
+    work-groups up to 512 (16-row block, KV head) items and two or three of
+    them together beyond (four always apart):
     a chunk of 41 rows (a ragged last block) at position 500 (36 pages for
     eight page streams) alone (9 items) and beside nine sequences of 304
     rows (522 items) gives bit-identical logits, within 1e-3 relative of the

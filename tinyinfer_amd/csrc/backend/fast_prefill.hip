@@ -53,12 +53,17 @@ namespace {
 constexpr int kDim = 64;
 constexpr int kPage = 16;
 constexpr int kWaves = 8;  // wavefronts (= page streams) per work item, two per SIMD
-// Work items up to which every query head has a work-group of its own: with
-// few items the launch is bound by one work-group's walk over its pages (an
-// idle chip), beyond by the matrix cores, and then one K/V load serves all
-// heads. Apart against together: 73 vs 85 us at 384 items of about 1,300
-// tokens, 91 vs 92 at 480, 138 vs 137 at 768, and 322 vs 303 on average over
-// 768 items of up to 8,700 tokens.
+// Work items up to which every one of two or three query heads has a
+// work-group of its own: with few items the launch is bound by one
+// work-group's walk over its pages (an idle chip), beyond by the matrix cores,
+// and then one K/V load serves all heads. Apart against together with three
+// heads: 73 vs 85 us at 384 items of about 1,300 tokens, 91 vs 92 at 480, 138
+// vs 137 at 768, and 322 vs 303 on average over 768 items of up to 8,700
+// tokens. With two (whole one-layer steps): 98 vs 126 at 64 items of 3,200
+// tokens, 244 vs 245 at 512, 336 vs 339 at 768. Four heads are always apart:
+// in pairs 269 vs 264 at 384 items of 1,500 tokens, 572 vs 557 at 1,024, 865
+// vs 844 at 1,024 of 3,500; together 570 and 826 at the last two, but 281 at
+// the first and 408 vs 367 at 384 of 3,500.
 constexpr int kSplitItems = 512;
 constexpr float kScale = 0.125f;  // 1/sqrt(64)
 constexpr float kRescale = 16.0f;  // probabilities stay below e^16 before a rescale
@@ -273,10 +278,7 @@ hipError_t launch_fast_prefill(hipStream_t s, const float* qkv, int ldq, int hea
         if (split) launch<3, 1>(s, qkv, ldq, kv, layer, it, count, kv_heads, out, ldo);
         else launch<3, 3>(s, qkv, ldq, kv, layer, it, count, kv_heads, out, ldo);
         break;
-    default:
-        if (split) launch<4, 1>(s, qkv, ldq, kv, layer, it, count, kv_heads, out, ldo);
-        else launch<4, 2>(s, qkv, ldq, kv, layer, it, count, kv_heads, out, ldo);
-        break;
+    default: launch<4, 1>(s, qkv, ldq, kv, layer, it, count, kv_heads, out, ldo); break;
     }
     return hipGetLastError();
 }
