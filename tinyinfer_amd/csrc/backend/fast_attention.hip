@@ -320,11 +320,15 @@ __global__ __launch_bounds__(kSplitPages * 64) void fast_attention_short_kernel(
     const int32_t* table = it + 4;
     const int split = fast_attention_split(length);
     const int splits = (length + split - 1) / split;  // 1..kSplitPages
-    if (wave < splits) {
+    const uint64_t touch = (uint64_t)blockIdx.x * kSplitPages + wave;
+    if (wave >= splits) {
+        // So does a wavefront without a split.
+        const float touched = touch_weights(w, touch, lane);
+        asm volatile("" ::"v"(touched));
+    } else {
         float m[HG], l[HG], acc[HG];
         const int t0 = wave * split;
         const int n = min(split, length - t0);
-        const uint64_t touch = (uint64_t)blockIdx.x * kSplitPages + wave;
         if (n == 2 * kPage)  // whole 32-token splits: exactly their two pages
             attend_split<HG, PLAIN, 2>(qkv, ldq, kv, layer, w, table, row, kvh, head0, t0, n, touch, p_s[wave], m, l, acc);
         else
