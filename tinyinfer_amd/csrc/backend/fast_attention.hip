@@ -63,13 +63,16 @@ constexpr int kMaxPages = 16;    // pages of one split
 constexpr int kRing = 2;                           // pages in flight per wavefront
 constexpr int kItemsPerGroup = 4;
 constexpr int kMergeHeld = 16;  // splits per lane group whose partials the merge loads in one round
-// Query heads of short rows in work-groups of their own up to this many, one
-// per CU: a wavefront's chain over its pages is then one head's instead of G
-// heads', which is what a small batch waits for. Apart against together: 5.9
-// vs 8.2 us for one row of 191 tokens, 9.6 vs 11.0 for 16 rows (144 heads),
-// 11.0 vs 11.1 to 12.4 for 28 (252), but 16.1 vs 12.1 for 56 (504), where the
-// work-groups queue for CUs.
-constexpr int kShortApart = 256;
+// Query heads of short rows in work-groups of their own up to this many: a
+// wavefront's chain over its pages is then one head's instead of G heads',
+// which is what a small batch waits for. Apart against together: 5.9 vs 8.2 us
+// for one row of 191 tokens, 9.6 vs 11.0 for 16 rows (144 heads). Towards a
+// work-group per CU nothing is gained (11.0 vs 11.1 to 12.4 for 28 rows, 252
+// heads) and the work-groups that would only prefetch weights have no CU:
+// 8-layer steps of 8 rows of 60 tokens on 8 KV heads of four (256 heads, 33 MB
+// of weights a layer) 443 vs 422 us, 16 rows on 4 KV heads of four 295 vs 293;
+// beyond, work-groups queue for CUs (56 rows, 504 heads: 16.1 vs 12.1 us).
+constexpr int kShortApart = 192;
 constexpr float kScale = 0.125f;  // 1/sqrt(64)
 constexpr float kRescale = 16.0f;  // probabilities stay below e^16 before a rescale
 
@@ -321,10 +324,11 @@ __global__ __launch_bounds__(kSplitPages * 64) void fast_attention_short_kernel(
     const int split = fast_attention_split(length);
     const int splits = (length + split - 1) / split;  // 1..kSplitPages
     const uint64_t touch = (uint64_t)blockIdx.x * kSplitPages + wave;
+    float touched = 0.0f;
     if (wave >= splits) {
-        // So does a wavefront without a split.
-        const float touched = touch_weights(w, touch, lane);
-        asm volatile("" ::"v"(touched));
+        // With the heads apart so does a wavefront without a split: there are
+        // G times as many work-groups with items, and fewer past them.
+        if (HG < G) touched = touch_weights(w, touch, lane);
     } else {
         float m[HG], l[HG], acc[HG];
         const int t0 = wave * split;
@@ -343,6 +347,7 @@ __global__ __launch_bounds__(kSplitPages * 64) void fast_attention_short_kernel(
         }
     }
     __syncthreads();
+    if (HG < G) asm volatile("" ::"v"(touched));
     if (wave >= HG) return;
     // Query head h: lane s < splits holds split s's (maximum, denominator)
     // (all in the first 16-lane row), lane d sums its dimension over the
