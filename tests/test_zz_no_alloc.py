@@ -197,3 +197,23 @@ def test_row_kernel_infinities_and_nans(torch_cuda, length):
                 ok = ~np.isnan(want)
                 assert np.array_equal(got[ok].view(np.uint32), want[ok].view(np.uint32)), (where, value, token)
                 assert np.all(np.isfinite(np.delete(got.reshape(KV_HEADS, -1), 1, axis=0)))
+
+
+@pytest.mark.parametrize("length", [77, 1500, 5000])
+def test_values_at_any_float(torch_cuda, length):
+    """V pools that start at any float, not only at 16 bytes: the oracle's
+    bits."""
+    torch, o = torch_cuda, Oracle()
+    q, keys, values, table = _inputs(o, 700, length)
+    want = o.attention(q, keys, values, table, length - 1, 1, LAYER, LAYERS, BT, HEADS, KV_HEADS, DIM)[0]
+    dq, dk, dt = (torch.from_numpy(a).cuda() for a in (q, keys, table))
+    for offset in (1, 2, 3):
+        room = torch.empty(values.size + 4, dtype=torch.float32, device="cuda")
+        dv = room[offset:offset + values.size]
+        dv.copy_(torch.from_numpy(values))
+        for call in (paged_attention_decode, paged_attention_decode_noalloc):
+            out = torch.zeros(HEADS * DIM, dtype=torch.float32, device="cuda")
+            call(dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dt.data_ptr(), length, LAYER, LAYERS, BT, HEADS, KV_HEADS,
+                 DIM, out.data_ptr(), None)
+            torch.cuda.synchronize()
+            assert np.array_equal(out.cpu().numpy().view(np.uint32), want.view(np.uint32)), (call.__name__, offset)

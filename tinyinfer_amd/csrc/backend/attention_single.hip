@@ -10,8 +10,9 @@
 // order is kept by ordered_sum.h with a whole wavefront.)
 //
 // Pages of 16 tokens with 64-wide heads take the kernels at the end of this
-// file (except where attention_row_pays says otherwise, and where out lies
-// over q); other shapes the general kernel below.
+// file (except where attention_row_pays says otherwise, where out lies over q
+// and where the values are not 16-byte aligned); other shapes the general
+// kernel below.
 #include "exact_math.h"
 #include "kernels.h"
 #include "layout.h"
@@ -580,7 +581,9 @@ hipError_t launch_attention_single(hipStream_t s, const float* q, const float* k
     // work-group touches them: such calls take it.
     const size_t width = (size_t)heads * dim;
     const bool over_q = (uintptr_t)out < (uintptr_t)(q + width) && (uintptr_t)q < (uintptr_t)(out + width);
-    if (block_tokens == kRowPage && dim == kRowDim &&
+    // The row kernel reads V in 16-byte pieces, the general kernel by floats.
+    const bool aligned = (uintptr_t)values % 16 == 0;
+    if (block_tokens == kRowPage && dim == kRowDim && aligned &&
         (scratch || (length <= kRowWindow && !over_q && attention_row_pays(heads, kv_heads, length)))) {
         const RowArgs a{q, keys, values, table, length, layer, layers, heads, kv_heads, out, scratch};
         switch (heads / kv_heads) {
